@@ -210,7 +210,7 @@ typedef struct raya_gemm_epilogue {
      *    row whose mean lies more than one standard deviation from zero is centred before
      *    the contraction, as ops::layer_norm subtracts the mean before scaling; for the
      *    others the mean comes out afterwards through the row sums.
-     * Both need the ring kernel: k a multiple of 16, lda, ldb, ldo (and ldr) multiples of
+     * Both need k a multiple of 16, lda, ldb, ldo (and ldr) multiples of
      * 4 floats, 16-byte aligned a, b and out (and residual); otherwise RAYA_ERR_UNSUPPORTED. */
     float *out_row_stats;
     const float *in_row_stats;

@@ -58,13 +58,13 @@ struct GemmLaunch {
     const float *rope_cos, *rope_sin;
     const int32_t *positions;
     int32_t rope_cols;
-    // A pre-LN LayerNorm of the input rows folded into the product (the ring
-    // kernel only): b holds the weight with the norm's gain folded into its
+    // A pre-LN LayerNorm of the input rows folded into the product (aligned rows and a
+    // depth that is a multiple of 16): b holds the weight with the norm's gain folded into its
     // columns, colsum[j] = sum_t b[j][t] (f64, rounded), and in_stats each row's
     // (mean_hi, mean_lo, rstd, 0) ([m], from launch_ln_stats; mean = mean_hi +
     // mean_lo, rstd = 1 / sqrt(var + eps)).  A row whose mean is more than one
-    // standard deviation from zero has its A operands centred by mean_hi as they
-    // leave LDS, so that its mean is removed before the contraction as
+    // standard deviation from zero has its A operands centred by mean_hi before they
+    // are split, so that its mean is removed before the contraction as
     // ops::layer_norm removes it before scaling; the rest of the mean comes out
     // as mean colsum.  Then y = rstd (acc - mean' colsum) before bias, activation
     // and RoPE: LayerNorm(a) W^T.  Null: off.
@@ -76,28 +76,24 @@ struct GemmLaunch {
     // mean as c + sum (x - c) / 64 to the precision of the deviations rather than
     // of |x|.  Null: off.
     float4 *out_stats;
-    // Split-K (the ring kernel only), for launches whose output tiles alone leave
-    // compute units idle: each tile's K loop is divided among `splits` workgroups,
-    // which store their partial tiles to `partials` ([tiles][splits][128 x 128]);
-    // a second launch of the same kernel (reduce = 1, set by launch_gemm) sums each
-    // tile's partials in split order and runs the epilogue.  splits <= 1: off.
+    // Split-K, for launches whose output tiles alone leave compute units idle: with
+    // room for them at `partials` (partial_floats floats; null: none), launch_gemm may
+    // divide each tile's K loop among workgroups that store their partial tiles there;
+    // a second launch of the same kernel sums each tile's partials in split order and
+    // runs the epilogue.
     float *partials;
-    int32_t splits;
-    int32_t reduce;
+    size_t partial_floats;
+    int32_t splits, reduce;  // set by launch_gemm
 };
 
-// Split-K for the ring kernel: the split count gemm_splits chooses for an
-// m x n output (GeGLU: n output columns from 2n weight rows) of depth k (1: no
-// split; never past kGemmSplitMaxTiles output tiles), and the partials' floats.
-constexpr int kGemmSplitMaxTiles = 256;
-int gemm_splits(int m, int n, int k, int act);
-size_t gemm_split_floats(int m, int n, int act, int splits);
+// The floats at GemmLaunch::partials that let launch_gemm split an m x n output (GeGLU: n
+// output columns from 2n weight rows) of depth k as it prefers (0: it would not).
+size_t gemm_partial_floats(int m, int n, int k, int act);
 
 // Head dim of the fused RoPE epilogue (other head dims use launch_rope).
 constexpr int kRopeHeadDim = 64;
 
 hipError_t launch_gemm(const GemmLaunch &g, hipStream_t stream);
-hipError_t launch_fill_zero(float *out, int64_t ldo, int m, int n, hipStream_t stream);
 
 // Row-wise LayerNorm over `rows` rows of width d (see encoder.hip).
 struct LayerNormLaunch {
@@ -128,7 +124,7 @@ hipError_t launch_gather_rows(const float *h, int64_t ldh, const int32_t *rows, 
 hipError_t launch_head_finish(const float *raw_logits, const uint8_t *mask, int batch, int markers,
                               const float *h, int64_t ldh, const int32_t *seq_start, int d,
                               float *logits, float *probs, float *features, float *pooled,
-                              float *act_in, int ld_act, hipStream_t stream);
+                              float *act_in, hipStream_t stream);
 
 // Thread-local error state of the C ABI (capi.cpp).
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -590,7 +590,6 @@ struct DeviceModel {
     DeviceBuf rope;  // global cos, global sin, local cos, local sin: [rope_len][head_dim / 2] each
     int rope_len = 0;
     DeviceBuf work;
-    DeviceBuf act_w;  // act_head.0.weight [256][d + 4] with its rows padded by zeros to ld_act
     FoldedNorms folded;
 };
 
@@ -631,27 +630,12 @@ int ensure_device(Model &m, DeviceModel **out) {
     return RAYA_OK;
 }
 
-int ensure_act_weight(const Model &m, DeviceModel &dm, uint64_t ld_act) {
-    if (dm.act_w.ptr) return RAYA_OK;
-    auto it = m.w.index.find("act_head.0.weight");
-    if (it == m.w.index.end()) return fail(RAYA_ERR_WEIGHTS, "missing act_head.0.weight");
-    const uint64_t k = m.cfg.hidden + 4, rows = 256;
-    const float *src = m.w.host.data() + m.w.entries[it->second].offset;
-    std::vector<float> host(rows * ld_act, 0.0f);
-    for (uint64_t r = 0; r < rows; ++r) memcpy(host.data() + r * ld_act, src + r * k, k * sizeof(float));
-    int rc = dm.act_w.reserve(host.size() * sizeof(float));
-    if (rc) return rc;
-    const hipError_t e = hipMemcpy(dm.act_w.ptr, host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return fail_device(e, "upload the padded act head weight");
-    return RAYA_OK;
-}
-
 // LN(x) W^T = rstd ((x - c) (g * W)^T - (mean - c) colsum) with g the norm's gain, colsum[j]
 // the row sums of g * W and c a per-row centre (0, or the mean's leading part for rows far
 // from zero; GemmLaunch::in_stats).  Built on the host once per device: the products
 // g_t W[j][t] in f32 (as LN's output times W rounds them) and their row sums in f64.  The
 // residual GEMMs that produce the statistics need whole 64-column chunks (hidden a multiple of
-// 64) and the ring kernel (every GEMM depth a multiple of 16: hidden and the MLP's intermediate
+// 64) and depths the kernels do not pad (multiples of 16: hidden and the MLP's intermediate
 // size); other shapes keep the LayerNorm kernels.
 bool norms_foldable(const Config &c) { return c.hidden % 64 == 0 && c.inter % 16 == 0; }
 
@@ -946,10 +930,6 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
 
     const uint64_t inter = c.inter, big = std::max(inter, c.head_ffn), nact = c.n_act;
     const uint64_t BK = B * K;
-    // The act head's first Linear has depth d + 4; its input rows and weight are padded with
-    // zeros to a multiple of 16 so that it runs on the ring kernel (and splits K).
-    const uint64_t ld_act = (d + 4 + 15) / 16 * 16;
-    if ((rc = ensure_act_weight(m, dm, ld_act))) return rc;
     // Split-K partials for the encoder GEMMs when the tokens are too few for their tiles to
     // fill the compute units (a single short sequence); other GEMMs split only if they fit.
     size_t split_cap = 0;
@@ -957,9 +937,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
         const uint64_t shapes[4][3] = {{3 * d, d, RAYA_EPI_NONE}, {d, d, RAYA_EPI_NONE}, {inter, d, RAYA_EPI_GEGLU},
                                        {d, inter, RAYA_EPI_NONE}};
         for (const auto &sh : shapes) {
-            const int act = (int)sh[2];
-            split_cap = std::max(split_cap, gemm_split_floats((int)T, (int)sh[0], act,
-                                                              gemm_splits((int)T, (int)sh[0], (int)sh[1], act)));
+            split_cap = std::max(split_cap, gemm_partial_floats((int)T, (int)sh[0], (int)sh[1], (int)sh[2]));
         }
     }
     size_t need = 0;
@@ -976,7 +954,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
         probe.take<float>(BK * 3);       // raw logits, logits, probabilities
         probe.take<float>(B * 4);        // features
         probe.take<float>(B * d);        // pooled
-        probe.take<float>(B * ld_act);   // act input, rows padded to the act head's depth
+        probe.take<float>(B * (d + 4));  // act input
         probe.take<float>(B * 256);      // act hidden
         probe.take<float>(B * nact);     // act logits
         probe.take<float4>(T * (d / 64));   // LayerNorm chunk statistics of h
@@ -995,7 +973,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
     float *raw = cv.take<float>(BK * 3);
     float *d_logits = raw + BK, *d_probs = raw + 2 * BK;
     float *d_feat = cv.take<float>(B * 4), *d_pooled = cv.take<float>(B * d);
-    float *act_in = cv.take<float>(B * ld_act), *act_hid = cv.take<float>(B * 256);
+    float *act_in = cv.take<float>(B * (d + 4)), *act_hid = cv.take<float>(B * 256);
     float *d_act = cv.take<float>(B * nact);
     float4 *hstats = cv.take<float4>(T * (d / 64));
     float4 *hrow = cv.take<float4>(T);
@@ -1077,16 +1055,11 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
 #define SPAN_END(slot) RECORD(span_end(slot))
 
     auto P = [&](const std::string &name) { return param(m, dm, name); };
-    // Split-K for a ring-kernel launch whose tiles leave compute units idle, when its
-    // partials fit the carved space (the launches run in order on one stream and share it).
+    // Every GEMM may split its depth within the carved space (the launches run in order on
+    // one stream and share it).
     auto set_split = [&](GemmLaunch &g) {
-        const bool ring = g.k % 16 == 0 && g.lda % 4 == 0 && g.ldb % 4 == 0 && ((uintptr_t)g.a & 15) == 0 &&
-                          ((uintptr_t)g.b & 15) == 0;
-        const int sp = ring ? gemm_splits(g.m, g.n, g.k, g.act) : 1;
-        if (sp > 1 && gemm_split_floats(g.m, g.n, g.act, sp) <= split_cap) {
-            g.splits = sp;
-            g.partials = partials;
-        }
+        g.partials = split_cap ? partials : nullptr;
+        g.partial_floats = split_cap;
     };
     auto gemm = [&](float *o, int64_t ldo, const float *a, int64_t lda, const float *wt, uint64_t rows, uint64_t n,
                     uint64_t k, int act, const float *bias, const float *res) -> int {
@@ -1333,13 +1306,13 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
     RECORD(gemm(s_hid, d, s_norm, d, P("scorer.1.weight"), BK, d, d, RAYA_EPI_GELU, P("scorer.1.bias"), nullptr));
     RECORD(gemm(raw, 1, s_hid, d, P("scorer.3.weight"), BK, 1, d, RAYA_EPI_NONE, P("scorer.3.bias"), nullptr));
     TRY_HIP(launch_head_finish(raw, d_mask, (int)B, (int)K, h, (int64_t)d, d_start, (int)d, d_logits, d_probs, d_feat,
-                               d_pooled, act_in, (int)ld_act, stream),
+                               d_pooled, act_in, stream),
             "head finish");
     RECORD(record_dense("logits", d_logits, {B, K}));
     RECORD(record_dense("probabilities", d_probs, {B, K}));
     RECORD(record_dense("act_features", d_feat, {B, 4}));
     RECORD(record_dense("pooled", d_pooled, {B, d}));
-    RECORD(gemm(act_hid, 256, act_in, ld_act, (const float *)dm.act_w.ptr, B, 256, ld_act, RAYA_EPI_GELU,
+    RECORD(gemm(act_hid, 256, act_in, d + 4, P("act_head.0.weight"), B, 256, d + 4, RAYA_EPI_GELU,
                 P("act_head.0.bias"), nullptr));
     RECORD(gemm(d_act, nact, act_hid, 256, P("act_head.2.weight"), B, nact, 256, RAYA_EPI_NONE, P("act_head.2.bias"),
                 nullptr));

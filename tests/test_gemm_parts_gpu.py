@@ -1,0 +1,108 @@
+"""The GEMM's three-part bfloat16 products where they can go wrong: the edges of every tile,
+depths that a slab does not divide, unaligned rows, operands of very different sizes, and operands
+whose parts do not sum to them (Inf, NaN, values above the largest bfloat16).
+
+Bar: the reordering bound 2 k 2^-24 sum |a b| around the float64 product
+(specs/009-gemm-backend-comparison/spec.md:24), which the sequential fp32 result meets.  The six
+part products leave out at most 2^-24 of a product and are summed smallest first, with 6
+roundings per 16 k, so they meet it for every k >= 1.  Non-finite results are compared with
+Reference::matmul_nt's.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from raya_amd import _capi as C
+
+pytestmark = pytest.mark.gpu
+
+GEGLU = C.RAYA_EPI_GEGLU
+
+
+def check(out, a, b):
+    k = a.shape[1]
+    a64, b64 = a.double(), b.double()
+    want = a64 @ b64.T
+    bound = 2 * k * 2.0 ** -24 * (a64.abs() @ b64.abs().T)
+    worst = float(((out.double() - want).abs() - bound).max())
+    assert worst <= 0, worst
+
+
+# Shapes by the tile they take: 32 x 64, 64 x 64, 64 x 128, 128 x 128, 256 x 128, 256 x 256, each one
+# row and column short of a whole tile or past it, with whole and padded depths.
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (33, 65, 128), (31, 63, 200), (257, 65, 15), (257, 2303, 768),
+                                   (321, 2177, 744), (513, 2305, 768), (511, 2303, 780), (1023, 2305, 768),
+                                   (1025, 2049, 100), (2047, 2305, 768), (2100, 2300, 720), (4097, 3073, 768),
+                                   (8193, 2300, 64)])
+def test_tile_edges(hip_gemm, m, n, k):
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    a = torch.randn(m, k, device="cuda", generator=gen)
+    b = torch.randn(n, k, device="cuda", generator=gen)
+    out = torch.full((m, n + 3), 9.0, device="cuda")
+    hip_gemm.matmul_nt_device(out[:, :n], a, b)
+    check(out[:, :n], a, b)
+    assert (out[:, n:] == 9.0).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 70, 131), (600, 500, 67), (5000, 777, 333)])
+def test_unaligned_rows(hip_gemm, m, n, k):
+    """Operand rows that start one float past a 16-byte boundary, at every alignment of the depth."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    for extra in range(4):
+        a = torch.randn(m, k + 1 + extra, device="cuda", generator=gen)[:, 1:k + 1]
+        b = torch.randn(n, k + 1 + extra, device="cuda", generator=gen)[:, 1:k + 1]
+        out = torch.empty(m, n, device="cuda")
+        hip_gemm.matmul_nt_device(out, a, b)
+        check(out, a, b)
+
+
+@pytest.mark.parametrize("m,n,k", [(50, 70, 96), (2100, 2300, 128)])
+def test_operands_over_the_whole_exponent_range(hip_gemm, m, n, k):
+    """Elements from 2^-60 to 2^60 in one row: each part keeps the operand's own exponent, so the
+    bound holds element by element, also where only a row's smallest elements meet b."""
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    scale = 2.0 ** torch.randint(-60, 61, (m, k), device="cuda", generator=gen)
+    a = torch.randn(m, k, device="cuda", generator=gen) * scale
+    b = torch.randn(n, k, device="cuda", generator=gen)
+    b[::2] *= (scale[:1] < 1).float()  # every other row of b meets the small half of a's first row only
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, a, b)
+    check(out, a, b)
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 70, 96), (300, 200, 100), (2100, 2300, 64)])
+def test_non_finite_operands(hip_gemm, m, n, k):
+    """Inf, NaN and 3.4e38 in single elements of a and b: NaN and Inf where the reference has
+    them, its values (the bound) elsewhere, and the outputs that meet none of them unchanged.
+    The two huge values share a column, so that an output's exact sum overflows whenever one of
+    its products does: where two huge products cancel, a sum overflows or not by its order."""
+    rng = np.random.default_rng(k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    b = rng.standard_normal((n, k)).astype(np.float32)
+    b[3, 5] = 0.0  # 0 * Inf
+    plain = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(plain, torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda())
+    x, y = a.copy(), b.copy()
+    for row, col, v in ((0, 5, np.inf), (7, k - 1, -np.inf), (m - 1, 0, np.nan), (33, 2, 3.4e38)):
+        x[row, col] = v
+    for row, col, v in ((1, 4, np.inf), (n - 1, k - 2, np.nan), (35, 2, -3.4e38)):
+        y[row, col] = v
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda())
+    got = out.cpu().numpy()
+    rows, cols = [0, 7, 33, m - 1], [1, 35, n - 1]
+    with np.errstate(all="ignore"):
+        for i, j in [(r, slice(None)) for r in rows] + [(slice(None), c) for c in cols]:
+            xa, yb = (x[i:i + 1], y) if isinstance(i, int) else (x, y[j:j + 1])
+            want = oracle.matmul_nt(np.ascontiguousarray(xa), np.ascontiguousarray(yb)).reshape(-1)
+            have = got[i, j].reshape(-1)
+            assert np.array_equal(np.isnan(have), np.isnan(want))
+            assert np.array_equal(have[np.isinf(want)], want[np.isinf(want)])
+            ok = np.isfinite(want)
+            bound = 2 * k * 2.0 ** -24 * (np.abs(xa).astype(np.float64) @ np.abs(yb).astype(np.float64).T).reshape(-1)
+            assert (np.abs(have[ok].astype(np.float64) - want[ok]) <= bound[ok]).all()
+    keep = np.ones((m, n), bool)
+    keep[rows] = False
+    keep[:, cols] = False
+    assert np.array_equal(got[keep], plain.cpu().numpy()[keep])
