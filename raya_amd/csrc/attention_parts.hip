@@ -1,0 +1,410 @@
+// Attention at head_dim 64 on three-part bfloat16 products: 128 query rows per workgroup.
+//
+// The fp32 matrix instruction bounds the multi-tile masks (Block3 at 16 x 8192 rows ran at
+// 113 of its 155 TFLOP/s).  Here every operand of both products is the exact sum of three
+// bfloat16 parts and a product the six part products that carry it, as in gemm_kernel.hpp:
+// 6 / 16 of the fp32 instruction's time, fewer roundings, and the probabilities keep all their
+// 24 bits.  Splitting costs 5.5 VALU operations an element, so a workgroup takes 128 rows:
+// each K and V element is split once for all of them, and each wave's 32 rows fill the
+// 32 x 32 x 16 instruction.  A wave's tile of 64 keys is 96 matrix instructions (3,072 clocks)
+// and about 500 VALU operations (2,400 at the 4.7 clocks they sustain); two waves a SIMD overlap
+// them to about 3,900 clocks a tile.
+//
+// Measured (us, before on the 64-row fp32 kernel): Block3 16 x 8192 116 -> 77 (165 TFLOP/s),
+// Block3 32 x 12 x 2048 402 -> 300, Full 4 x 12 x 2048 (1024 to 2048 valid) 342 -> 219, Full
+// 1 x 12 x 4096 442 -> 294 (175 TFLOP/s); relative 2-norm error against float64 4.6e-7 -> 3.9e-7
+// (Block3), 7.7e-7 -> 7.0e-7 (Full).
+//
+//   S^T = K Q^T (32 keys x 32 queries per subtile), online softmax as in attention_body.hpp,
+//   O^T += V^T P^T, P^T taken straight from the S^T registers.
+//
+// Layouts of v_mfma_f32_32x32x16_bf16 (lane l, li = l % 32, h = l / 32): A[li][8h + e],
+// B[8h + e][li] for e = 0 .. 7, D[8 (r / 4) + 4h + r % 4][li] in register r.  The score of key
+// 8 (r / 4) + 4h + r % 4 of a subtile is register r, so registers 8s .. 8s + 7 are the
+// B operand of PV step s when its contraction index (h, e) is key 16s + 8 (e / 4) + 4h + e % 4;
+// V is written to LDS transposed in that order.
+//
+// LDS holds one tile of 64 keys: K's parts while the scores are formed, V's while they are
+// used.  Phase A forms the scores of tile j while V of tile j is split into place, phase B takes
+// the softmax and PV while K of tile j + 1 is: the VALU work of the splitting runs beside the
+// matrix cores, with one barrier after each phase.  Rows are fetched into registers two phases
+// ahead.
+//
+// Outputs that are not finite (an operand that is not finite, or above the largest bfloat16,
+// has no parts) are computed again by the fp32 body in the same workgroup, and only they.
+#include "attention_body.hpp"
+#include "parts.hpp"
+
+namespace raya {
+namespace attn {
+namespace {
+
+// acc[i] += a[i] b over the parts, the smallest products first; the two sums alternate, so that
+// no instruction waits for the one before it.
+__device__ __forceinline__ void products(const bf16x8 (&a)[2][3], const bf16x8 (&b)[3], floatx16 (&acc)[2]) {
+    constexpr int qa[6] = {2, 0, 1, 1, 0, 0}, qb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i] = mfma_bf16(a[i][qa[q]], b[qb[q]], acc[i]);
+}
+__device__ __forceinline__ void product(const bf16x8 (&a)[3], const bf16x8 (&b)[3], floatx16 &acc) {
+    constexpr int qa[6] = {2, 0, 1, 1, 0, 0}, qb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+    for (int q = 0; q < 6; ++q) acc = mfma_bf16(a[qa[q]], b[qb[q]], acc);
+}
+
+constexpr int D = 64, DS = D / 16, DT = D / 32;  // head_dim, its MFMA steps and 32-wide tiles
+constexpr int kPlane = kKeys * D * 2;            // bytes of one part of a K or V tile
+constexpr int kPartTile = 3 * kPlane;
+
+// K part blocks: [32-key subtile][step][h][32 keys][8 dims]; key row r of the block at slot
+// r ^ (2 step + h), so that the 16 lanes that write one row's chunks cover 128 bytes.
+__device__ __forceinline__ int k_slot(int key, int step, int h) {
+    return ((key >> 5) * DS + step) * 1024 + h * 512 + ((key & 31) ^ (2 * step + h)) * 16;
+}
+// V part blocks: [32-dim tile][16-key step][h][32 dims][8 keys]; dim row d at slot
+// d ^ ((d / 4) & 7), so that 8 lanes writing dims 4 apart hit 8 different slots mod 8.
+__device__ __forceinline__ int v_slot(int dim, int step, int h) {
+    const int d = dim & 31;
+    return ((dim >> 5) * (kKeys / 16) + step) * 1024 + h * 512 + (d ^ ((d >> 2) & 7)) * 16;
+}
+
+template <int MK, bool TIMED>
+__device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, char *lds, StageClock *clk) {
+    // Windows leave each wave whole subtiles outside its rows' keys; the block masks' items see
+    // every key of their range.
+    constexpr bool WINDOW = MK == RAYA_MASK_SLIDING;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int li = lane & 31, h = lane >> 5;
+    const Item it = decode<kPartRows, MK>(a, p, item_of(blockIdx.x, p));
+    const bool packed = a.seq_start != nullptr;
+    const int64_t row0 = packed ? (int64_t)a.seq_start[it.b] : 0;
+    const auto base = [&](int64_t bs, int64_t hs, int64_t rs) {
+        return (packed ? row0 * rs : (int64_t)it.b * bs) + (int64_t)it.h * hs;
+    };
+    float *ob = a.out + base(a.o_bs, a.o_hs, a.o_rs);
+    if (it.k_lo >= it.k_hi) {  // every row is padding: write zeros
+        if (packed) return;
+        for (int c = tid; c < kPartRows * 16; c += kThreads) {
+            const int r = it.q0 + c / 16;
+            if (r < a.seq) store_stream(ob + (int64_t)r * a.o_rs + 4 * (c % 16), make_float4(0.f, 0.f, 0.f, 0.f));
+        }
+        return;
+    }
+    const float c_exp = fmaxf(fabsf(a.scale) * kLog2e, 1.17549435e-38f);
+    const float q_sign = a.scale < 0.f ? -1.f : 1.f;
+    const int valid = it.valid, arg = a.mask_arg;
+    const int qw = it.q0 + 32 * wave, qi = qw + li;
+    const Range rr = qi < valid ? key_range(MK, arg, p.by_arg, qi, valid) : Range{0, 0};
+    const bool wave_live = qw < valid, wave_full = qw + 31 < valid;
+    const Range w_first = key_range(MK, arg, p.by_arg, min(qw, valid - 1), valid);
+    const Range w_last = key_range(MK, arg, p.by_arg, min(qw + 31, valid - 1), valid);
+    const float *kb = a.k + base(a.k_bs, a.k_hs, a.k_rs), *vb = a.v + base(a.v_bs, a.v_hs, a.v_rs);
+
+    // The item's tiles, walked from the one whose index is a multiple of their count
+    // (attention_body.hpp: neighbours' first touches spread over the steps).
+    const int n_tiles = (it.k_hi - it.k_lo + kKeys - 1) / kKeys;
+    int rot = (it.k_lo / kKeys) % n_tiles;
+    rot = rot == 0 ? 0 : n_tiles - rot;
+    const auto tile_at = [&](int j) {
+        j += rot;
+        return it.k_lo + (j >= n_tiles ? j - n_tiles : j) * kKeys;
+    };
+
+    // Staging.  K: 16 lanes take a row's 16-byte chunks, 16 rows a pass.  V: each thread takes 4
+    // keys x 4 dims (key quad 4 s + 2 half + vh of PV step s), so that it can write 4 keys of a
+    // dim together.
+    const int kc = tid & 15, kr = tid >> 4;
+    const int vs = wave, half = (lane >> 3) & 1, vh = (lane >> 4) & 1, dq = (lane & 7) + 8 * (lane >> 5);
+    const int vkey = 16 * vs + 8 * half + 4 * vh;
+    float4 kreg[4], vreg[4];
+    // Keys past the item's last one are fetched as copies of it.
+    const auto load_k = [&](int j) {
+        const int kt = tile_at(min(j, n_tiles - 1)), last = it.k_hi - 1 - kt;
+        const float *src = kb + (int64_t)kt * a.k_rs;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            kreg[i] = *(const float4 *)(src + (uint32_t)(min(kr + 16 * i, last) * (int)a.k_rs) + 4 * kc);
+    };
+    const auto load_v = [&](int j) {
+        const int kt = tile_at(min(j, n_tiles - 1)), last = it.k_hi - 1 - kt;
+        const float *src = vb + (int64_t)kt * a.v_rs;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            vreg[i] = *(const float4 *)(src + (uint32_t)(min(vkey + i, last) * (int)a.v_rs) + 4 * dq);
+    };
+    char *kl = lds, *vl = lds + kPartTile;
+    const auto put_k = [&](int i) {
+        uint32_t lo[3], hi[3];
+        split3(kreg[i].x, kreg[i].y, lo);
+        split3(kreg[i].z, kreg[i].w, hi);
+        char *d = kl + k_slot(kr + 16 * i, kc >> 2, (kc >> 1) & 1) + (kc & 1) * 8;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * kPlane) = uint32x2{lo[q], hi[q]};
+    };
+    // Dim 4 dq + i of this thread's four keys.
+    const auto put_v = [&](int i) {
+        const auto at = [&](int k) {
+            const float4 &x = vreg[k];
+            return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w;
+        };
+        uint32_t lo[3], hi[3];
+        split3(at(0), at(1), lo);
+        split3(at(2), at(3), hi);
+        char *d = vl + v_slot(4 * dq + i, vs, vh) + half * 8;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * kPlane) = uint32x2{lo[q], hi[q]};
+    };
+
+    load_k(0);
+    load_v(0);
+    // Q's parts: dims 16 s + 8 h .. + 7 of this lane's row (rows at or beyond valid take the last
+    // one's, and all their keys are masked), negated for a negative scale.
+    bf16x8 qf[DS][3];
+    {
+        const float *qp = a.q + base(a.q_bs, a.q_hs, a.q_rs) + (int64_t)min(qi, valid - 1) * a.q_rs + 8 * h;
+#pragma unroll
+        for (int s = 0; s < DS; ++s) {
+            const float4 x = *(const float4 *)(qp + 16 * s), y = *(const float4 *)(qp + 16 * s + 4);
+            const float e[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+            uint32x4 w[3];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                uint32_t part[3];
+                split3(e[2 * c] * q_sign, e[2 * c + 1] * q_sign, part);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) w[q][c] = part[q];
+            }
+#pragma unroll
+            for (int q = 0; q < 3; ++q) qf[s][q] = __builtin_bit_cast(bf16x8, w[q]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) put_k(i);
+    load_k(1);
+    __syncthreads();
+
+    floatx16 oacc[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[t][r] = 0.f;
+    float m = -INFINITY;  // running max of the scores times c_exp, rounded: the weights' reference
+    float l = 0.f;        // this lane's partial sum of weights
+    if constexpr (TIMED) clk->last = clock_now();
+
+#pragma unroll 1
+    for (int j = 0; j < n_tiles; ++j) {
+        const int kt = tile_at(j);
+        int live = wave_live ? 3 : 0;  // subtiles with a key of some row of the wave
+        if constexpr (WINDOW) {
+            live = 0;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                if (wave_live && kt + 32 * t < w_last.hi && kt + 32 * t + 32 > w_first.lo) live |= 1 << t;
+        }
+        // Phase A: scores.
+        floatx16 s[2];
+        if constexpr (TIMED) clk->tiles += live ? (wave_full || qw + 16 < valid ? 2 : 1) : 0;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
+        if constexpr (WINDOW) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (live >> t & 1) {
+#pragma unroll
+                    for (int d = 0; d < DS; ++d) {
+                        bf16x8 kf[3];
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            kf[q] = *(const bf16x8 *)(kl + q * kPlane + k_slot(32 * t + li, d, h));
+                        product(kf, qf[d], s[t]);
+                    }
+                }
+                put_v(2 * t);
+                put_v(2 * t + 1);
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < DS; ++d) {
+                bf16x8 kf[2][3];
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int q = 0; q < 3; ++q)
+                        kf[t][q] = *(const bf16x8 *)(kl + q * kPlane + k_slot(32 * t + li, d, h));
+                products(kf, qf[d], s);
+                put_v(d);
+            }
+        }
+        load_v(j + 1);
+        if constexpr (TIMED) {
+            settle(s[0][15]);
+            settle(s[1][15]);
+            lap(clk, clk->qk);
+        }
+        __syncthreads();
+        if constexpr (TIMED) lap(clk, clk->load_wait);
+
+        // Phase B: the softmax update, then PV.
+        if (!WINDOW || live) {
+            if (WINDOW || !(wave_full && kt >= w_last.lo && kt + kKeys <= w_first.hi)) {
+                const int lo = rr.lo - kt - 4 * h, hi = rr.hi - kt - 4 * h;
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int key = 32 * t + 8 * (r >> 2) + (r & 3);
+                        if (key < lo || key >= hi || (WINDOW && !(live >> t & 1))) s[t][r] = -INFINITY;
+                    }
+            }
+            float tmax = s[0][0];
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[t][r]);
+            tmax = max_xor32(tmax);
+            const float m_new = fmaxf(m, tmax * c_exp);
+            const float m_use = m_new == -INFINITY ? 0.f : m_new;
+            if (__any(m_new > m)) {  // otherwise every factor is 1
+                const float alpha = fast_exp2(m - m_use);
+                l *= alpha;
+#pragma unroll
+                for (int t = 0; t < DT; ++t) oacc[t] *= alpha;
+            }
+            m = m_new;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (WINDOW && !(live >> t & 1)) continue;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    s[t][r] = fast_exp2(__builtin_fmaf(s[t][r], c_exp, -m_use));
+                    l += s[t][r];
+                }
+            }
+            if constexpr (TIMED) {
+                settle(l);
+                settle(oacc[0][15]);
+                lap(clk, clk->softmax);
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            if (!WINDOW || (live >> t & 1)) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    uint32x4 w[3];
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        uint32_t part[3];
+                        split3(s[t][8 * u + 2 * c], s[t][8 * u + 2 * c + 1], part);
+#pragma unroll
+                        for (int q = 0; q < 3; ++q) w[q][c] = part[q];
+                    }
+                    bf16x8 pf[3], vf[DT][3];
+#pragma unroll
+                    for (int q = 0; q < 3; ++q) pf[q] = __builtin_bit_cast(bf16x8, w[q]);
+#pragma unroll
+                    for (int d = 0; d < DT; ++d)
+#pragma unroll
+                        for (int q = 0; q < 3; ++q)
+                            vf[d][q] = *(const bf16x8 *)(vl + q * kPlane + v_slot(32 * d + li, 2 * t + u, h));
+                    products(vf, pf, oacc);
+                }
+            }
+            put_k(2 * t);
+            put_k(2 * t + 1);
+        }
+        load_k(j + 2);
+        if constexpr (TIMED) {
+            settle(oacc[0][15]);
+            settle(oacc[1][15]);
+            lap(clk, clk->pv);
+        }
+        __syncthreads();
+        if constexpr (TIMED) lap(clk, clk->load_wait);
+    }
+
+    // Dims 32 t + 8 r + 4 h .. + 3 of row qi are registers 4 r .. 4 r + 3 of oacc[t].  Each
+    // wave's 32 x 64 outputs go through LDS and leave as whole rows (attention_body.hpp).
+    l = sum_xor32(l);
+    float *st = (float *)lds + wave * 32 * D;
+    const bool zero_row = qi >= valid || l == 0.f;
+    const float inv = zero_row ? 0.f : 1.f / l;
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (!zero_row)
+                y = make_float4(oacc[t][4 * r] * inv, oacc[t][4 * r + 1] * inv, oacc[t][4 * r + 2] * inv,
+                                oacc[t][4 * r + 3] * inv);
+            bad |= !finite4(y);
+            *(float4 *)(st + li * D + 4 * ((8 * t + 2 * r + h) ^ (li & 15))) = y;
+        }
+    const int rows = packed ? valid : a.seq;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = 4 * i + (lane >> 4), c = lane & 15;
+        const float4 y = *(const float4 *)(st + r * D + 4 * (c ^ (r & 15)));
+        if (qw + r < rows) store_stream(ob + (int64_t)(qw + r) * a.o_rs + 4 * c, y);
+    }
+    if (__syncthreads_or(bad)) {
+        // (The barrier's fence has the stores done and the staging read.)
+        __threadfence();
+#pragma unroll 1
+        for (int q0 = it.q0; q0 < min(it.q0 + kPartRows, valid); q0 += kQRows) {
+            Item half_item = it;
+            half_item.q0 = q0;
+            half_item.k_lo = key_range(MK, arg, p.by_arg, q0, valid).lo;
+            half_item.k_hi = key_range(MK, arg, p.by_arg, min(q0 + kQRows, valid) - 1, valid).hi;
+            attend_body<D, true, false, WINDOW, false, MK, false, 0, WINDOW, true>(a, p, half_item, (float *)lds,
+                                                                                  (float *)lds + kKeys * D, nullptr);
+            __syncthreads();
+        }
+    }
+}
+
+template <int MK>
+__global__ void __launch_bounds__(kThreads, 2) attend_parts_kernel(const AttnLaunch a, const Plan p) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile];
+    parts_body<MK, false>(a, p, lds, nullptr);
+}
+
+// The same with the stage clock (attention.hip's attend_timed_kernel).
+template <int MK>
+__global__ void __launch_bounds__(kThreads, 2) attend_parts_timed_kernel(const AttnLaunch a, const Plan p) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile];
+    __shared__ uint64_t part[kWaves][5];
+    StageClock c{};
+    parts_body<MK, true>(a, p, lds, &c);
+    add_stage_totals(a, c, part);
+}
+
+template <int MK>
+void launch_mask(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
+    const dim3 grid((unsigned)p.total), block(kThreads);
+    if (a.stage_cycles)
+        hipLaunchKernelGGL((attend_parts_timed_kernel<MK>), grid, block, 0, stream, a, p);
+    else
+        hipLaunchKernelGGL((attend_parts_kernel<MK>), grid, block, 0, stream, a, p);
+}
+
+}  // namespace
+
+hipError_t launch_parts(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
+    switch (a.mask_kind) {
+    case RAYA_MASK_BLOCK3: launch_mask<RAYA_MASK_BLOCK3>(a, p, stream); break;
+    case RAYA_MASK_FULL: launch_mask<RAYA_MASK_FULL>(a, p, stream); break;
+    case RAYA_MASK_SLIDING: launch_mask<RAYA_MASK_SLIDING>(a, p, stream); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace attn
+}  // namespace raya

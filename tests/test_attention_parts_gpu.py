@@ -1,0 +1,154 @@
+"""The 128-row attention kernel on three-part bfloat16 products, forced with RAYA_ATTN_ITEMS=128:
+edges of its tiles and waves under every mask it takes, strided and padded batches, non-finite
+operands, and its instrumented copy.
+
+Bars as in test_attention_gpu.py: max-abs 1e-5 and rel-L2 1e-5 against the oracle's Naive (an fp32
+reordering bar; the parts carry all 24 bits of every operand), exact zeros on padded rows.
+"""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import raya_amd as R
+from raya_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+MASKS = {"block3": (R.Mask.BLOCK3, oracle.MASK_BLOCK3, 128, 0), "full": (R.Mask.FULL, oracle.MASK_FULL, 0, 0),
+         "sliding64": (R.Mask.sliding(64), oracle.MASK_SLIDING, 0, 64),
+         "sliding7": (R.Mask.sliding(7), oracle.MASK_SLIDING, 0, 7),
+         "sliding200": (R.Mask.sliding(200), oracle.MASK_SLIDING, 0, 200)}
+
+
+@pytest.fixture(autouse=True)
+def items128(monkeypatch):
+    monkeypatch.setenv("RAYA_ATTN_ITEMS", "128")
+
+
+def inputs(seed, h, s, d=64):
+    return [synth.normal(1000 * seed + i, h * s * d).reshape(h, s, d) for i in range(3)]
+
+
+def naive(q, k, v, name, valid, scale=0.125):
+    _, kind, block, window = MASKS[name]
+    return oracle.naive_attend(q, k, v, kind, valid, scale, block=block, window=window)
+
+
+def close(got, want):
+    assert np.isfinite(got).all()
+    diff = np.abs(got - want)
+    assert diff.max() <= 1e-5, diff.max()
+    assert np.sqrt((diff.astype(np.float64) ** 2).sum()) <= 1e-5 * np.sqrt((want.astype(np.float64) ** 2).sum())
+
+
+@pytest.mark.parametrize("name", list(MASKS))
+@pytest.mark.parametrize("seq", [1, 31, 33, 64, 127, 129, 300, 513])
+def test_edges(hip_attention, name, seq):
+    """One launch of sequences whose valid lengths end at, before and after every kind of edge."""
+    h = 2
+    lens = sorted({max(0, min(seq, n)) for n in (0, 1, 16, 32, 65, 128, 130, 257, seq - 1, seq)})
+    qkv = [inputs(100 + n, h, seq) for n in range(len(lens))]
+    dev = [torch.from_numpy(np.stack([x[i] for x in qkv])).cuda() for i in range(3)]
+    out = torch.full_like(dev[0], 7.0)
+    print(f"{name} seq {seq} lens {lens}", flush=True)
+    hip_attention.attend_batched(*dev, out, torch.tensor(lens, dtype=torch.int32, device="cuda"), MASKS[name][0])
+    got = out.cpu().numpy()
+    for b, n in enumerate(lens):
+        assert (got[b, :, n:] == 0).all()
+        if n:
+            close(got[b, :, :n], naive(*qkv[b], name, n)[:, :n])
+
+
+@pytest.mark.parametrize("name", ["block3", "full", "sliding64"])
+@pytest.mark.parametrize("scale", [-0.2, 0.0, 0.125])
+def test_packed_projection_and_scales(hip_attention, name, scale):
+    """Heads read out of a [batch][seq][3 heads dim] projection with padded rows between."""
+    b, h, s, d, pad = 2, 3, 260, 64, 8
+    width = 3 * h * d + pad
+    rows = torch.from_numpy(synth.normal(77, b * s * width).reshape(b, s, width)).cuda()
+    out = torch.full((b, s, h * d + 4), 9.0, device="cuda")
+    lay = (s * width, d, width)
+    hip_attention.attend_batched(rows, rows[:, :, h * d:], rows[:, :, 2 * h * d:], out,
+                                 torch.tensor([s, 200], dtype=torch.int32, device="cuda"), MASKS[name][0], scale,
+                                 layouts={"shape": (b, h, s, d), "q": lay, "k": lay, "v": lay,
+                                          "out": (s * (h * d + 4), d, h * d + 4)})
+    got, x = out.cpu().numpy(), rows.cpu().numpy()
+    assert (got[:, :, h * d:] == 9.0).all()
+    for i, n in enumerate((s, 200)):
+        q, k, v = (np.ascontiguousarray(x[i, :, j * h * d:(j + 1) * h * d].reshape(s, h, d).transpose(1, 0, 2))
+                   for j in range(3))
+        have = got[i, :, :h * d].reshape(s, h, d).transpose(1, 0, 2)
+        assert (have[:, n:] == 0).all()
+        close(have[:, :n], naive(q, k, v, name, n, scale)[:, :n])
+
+
+@pytest.mark.parametrize("name", list(MASKS))
+@pytest.mark.parametrize("operand", [0, 1, 2])
+def test_non_finite_operands_match_the_reference(hip_attention, name, operand):
+    """Inf, -Inf, NaN and 3.4e38 in one row of q, k or v at a time: NaN and Inf where Naive has
+    them, its values elsewhere."""
+    h, s, valid = 1, 300, 290
+    for at, value in ((0, np.inf), (63, -np.inf), (130, np.nan), (valid - 1, -np.inf), (200, 3.4e38)):
+        x = inputs(9, h, s)
+        x[operand][0, at, 5] = value
+        with np.errstate(all="ignore"):
+            want = naive(*x, name, valid)
+        out = np.full(h * s * 64, 7.0, np.float32)
+        hip_attention.attend(R.AttnShape(h, s, 64), R.AttnParams(MASKS[name][0], 128, valid, 0.125),
+                             *(t.reshape(-1) for t in x), out)
+        got = out.reshape(want.shape)
+        assert np.array_equal(np.isnan(got), np.isnan(want)), (at, value)
+        assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)]), (at, value)
+        ok = np.isfinite(want)
+        assert (np.abs(got[ok] - want[ok]) <= 1e-5 * np.maximum(1.0, np.abs(want[ok]))).all(), (at, value)
+
+
+@pytest.mark.parametrize("name", ["block3", "full", "sliding64"])
+def test_error_is_no_larger_than_the_fp32_kernels(hip_attention, monkeypatch, name):
+    """RMS distance from float64 attention, against the 64-row kernel's on the fp32 instruction."""
+    h, s = 4, 1024
+    x = inputs(5, h, s)
+    dev = [torch.from_numpy(t[None]).cuda() for t in x]
+    valid = torch.tensor([s], dtype=torch.int32, device="cuda")
+    outs = {}
+    for items in ("128", "64"):
+        monkeypatch.setenv("RAYA_ATTN_ITEMS", items)
+        outs[items] = torch.empty_like(dev[0])
+        hip_attention.attend_batched(*dev, outs[items], valid, MASKS[name][0])
+    q, k, v = (t[0].double() for t in dev)
+    i = torch.arange(s, device="cuda")
+    seen = {"block3": (i[:, None] // 128 - i[None] // 128).abs() <= 1, "full": (i[:, None] >= 0) & (i[None] >= 0),
+            "sliding64": (i[:, None] - i[None]).abs() <= 64}[name]
+    w = torch.softmax((torch.matmul(q, k.transpose(1, 2).contiguous()) * 0.125).masked_fill(~seen, -np.inf), -1)
+    want = torch.matmul(w, v)
+    rms = {n: float(((o[0].double() - want) ** 2).mean().sqrt()) for n, o in outs.items()}
+    print(name, rms)
+    assert rms["128"] <= 1.05 * rms["64"]
+
+
+@pytest.mark.parametrize("name", ["block3", "sliding64"])
+def test_stages(hip_attention, name):
+    """The instrumented copy: the same outputs, the tiles of 16 rows x 64 keys it computes (two to
+    a wave of 32 rows that meets the tile, one if its second 16 are padding)."""
+    seq, heads, lens = 512, 2, [512, 300]
+    dev = [torch.from_numpy(np.stack([inputs(n, heads, seq)[i] for n in (1, 2)])).cuda() for i in range(3)]
+    valid = torch.tensor(lens, dtype=torch.int32, device="cuda")
+    mask = MASKS[name][0]
+    plain = torch.empty_like(dev[0])
+    hip_attention.attend_batched(*dev, plain, valid, mask)
+    timed = torch.empty_like(plain)
+    st = hip_attention.attend_batched_stages(*dev, timed, valid, mask)
+    assert torch.equal(timed, plain)
+    assert st.qk > 0 and st.softmax > 0 and st.pv > 0 and st.load_wait > 0
+    n = 0
+    for v in lens:
+        for q0 in range(0, v, 128):
+            lo = mask.key_range(q0, v).start
+            hi = mask.key_range(min(q0 + 128, v) - 1, v).stop
+            for kt in range(lo, hi, 64):
+                for w in range(q0, min(q0 + 128, v), 32):
+                    a, z = mask.key_range(w, v), mask.key_range(min(w + 31, v - 1), v)
+                    meets = any(t < z.stop and t + 32 > a.start for t in (kt, kt + 32))
+                    n += (2 if w + 16 < v else 1) if meets else 0
+    assert st.tiles == n * heads
