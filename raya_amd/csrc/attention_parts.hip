@@ -72,8 +72,10 @@ __device__ __forceinline__ int v_slot(int dim, int step, int h) {
 
 // Item `item` with the sequences taken longest first (ties in order).  Under Full an item's work
 // is its sequence's length, and a long one that starts last is waited for alone: 4 sequences of
-// 1024 to 2048 rows x 12 heads in the caller's order 219 us, longest first @@ us.  One lane a
-// sequence, so batches past 64 keep their order.
+// 1024 to 2048 rows x 12 heads in the caller's order 224 us, longest first 208; 8 of 100 to 300
+// rows 27.0 -> 22.4.  Batches past kMaxSorted keep their order: their tails are too short to pay
+// for the ranking (64 of 128 to 512 rows: 194 -> 198 us).
+constexpr int kMaxSorted = 16;
 __device__ __forceinline__ Item decode_longest_first(const AttnLaunch &a, const Plan &p, int item) {
     const int bh = fdiv(item, p.by_qt), slot = fdiv(bh, p.by_heads), lane = threadIdx.x & 63;
     const int mine = lane < a.batch ? min(max(a.valid_len[min(lane, a.batch - 1)], 0), a.seq) : -1;
@@ -94,7 +96,7 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int li = lane & 31, h = lane >> 5;
     const int item = item_of(blockIdx.x, p);
-    const bool sorted = MK == RAYA_MASK_FULL && a.valid_len && a.batch > 1 && a.batch <= 64;
+    const bool sorted = MK == RAYA_MASK_FULL && a.valid_len && a.batch > 1 && a.batch <= kMaxSorted;
     const Item it = sorted ? decode_longest_first(a, p, item) : decode<kPartRows, MK>(a, p, item);
     const bool packed = a.seq_start != nullptr;
     const int64_t row0 = packed ? (int64_t)a.seq_start[it.b] : 0;
