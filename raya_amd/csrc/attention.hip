@@ -99,7 +99,7 @@ int scatter_half_bits(int64_t total) {
 // split kernel runs 3 workgroups per compute unit).
 constexpr int64_t kSplitBelow = 192;
 
-// Whether a launch at head_dim 64 takes the 128-row kernel on three-part products
+// Whether a launch at head_dim 64 or 128 takes the 128-row kernel on three-part products
 // (attention_parts.hip), by the masks and grids where it is the faster one (us, 128-row / 64-row /
 // 16-row items, 12 heads unless said):
 // - Full and Block3: 16 x 8192 Block3 78 / 112; 4 x 2048 Full 217 / 322; sequences of 768
@@ -111,23 +111,27 @@ constexpr int64_t kSplitBelow = 192;
 //   40.6 / 34.1 / 29.8, 1 x 1536 41.2 / 50.1 / 44.9).
 // - not BlockDiag: one or two tiles an item leave nothing to gain from cheaper products (64 is
 //   bound by memory).
+// - head_dim 128 (one wave a SIMD: Q's parts and the output alone fill 160 registers): Block3
+//   2 x 8 x 3000 83 / 99, 8 x 8 x 2048 167 / 228, Full 2 x 8 x 2048 185 / 290; from 144 items (Block3
+//   1 x 8 x 1536, 96 items, 36.3 / 35.5), Sliding from w = 128 (64: 70.5 / 68.1, 128: 96 / 101).
 // Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.
 constexpr int64_t kPartsFrom = 144, kPartsFromWide = 72;
-constexpr int64_t kWideSeq = 384, kPartsWindow = 80;
+constexpr int64_t kWideSeq = 384, kPartsWindow = 80, kPartsWindow128 = 128;
 
 bool takes_parts(const AttnLaunch &a) {
     const bool block = a.mask_kind == RAYA_MASK_FULL || a.mask_kind == RAYA_MASK_BLOCK3;
-    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= kPartsWindow)) return false;
+    const bool wide = a.head_dim > 64;
+    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= (wide ? kPartsWindow128 : kPartsWindow))) return false;
     const int64_t tiles = (a.seq + kPartRows - 1) / kPartRows;
     if (5 * (int64_t)a.seq < 3 * kPartRows * tiles) return false;  // under 60% of the items' rows
-    return tiles * a.heads * a.batch >= (block && a.seq >= kWideSeq ? kPartsFromWide : kPartsFrom);
+    return tiles * a.heads * a.batch >= (block && !wide && a.seq >= kWideSeq ? kPartsFromWide : kPartsFrom);
 }
 
 // Query rows of an item.  RAYA_ATTN_ITEMS=16, 64 or 128 forces the height where the kernel
 // exists (as the reference's RAYA_BACKEND forces a micro-kernel backend); anything else selects
 // by grid.
-int64_t item_rows(const AttnLaunch &a, bool head64) {
-    const bool parts_ok = head64 && a.mask_kind != RAYA_MASK_BLOCKDIAG && a.mask_kind != RAYA_MASK_WINDOW64;
+int64_t item_rows(const AttnLaunch &a, bool parts_dim) {
+    const bool parts_ok = parts_dim && a.mask_kind != RAYA_MASK_BLOCKDIAG && a.mask_kind != RAYA_MASK_WINDOW64;
     if (const char *e = std::getenv("RAYA_ATTN_ITEMS")) {
         if (!std::strcmp(e, "16")) return kSplitRows;
         if (!std::strcmp(e, "64")) return kQRows;
@@ -208,7 +212,9 @@ void launch_split_all(int64_t t, dim3 grid, dim3 block, hipStream_t stream, cons
 
 template <int DP, bool FUSED = false>
 hipError_t launch_dp(const AttnLaunch &a, hipStream_t stream) {
-    const int64_t rows = item_rows(a, FUSED);
+    // (The same row strides as the fused issue's: the parts' rows are addressed within a tile too.)
+    constexpr bool PARTS = FUSED || DP == 128;
+    const int64_t rows = item_rows(a, PARTS && a.head_dim == DP && a.k_rs < kMaxFusedRowStride && a.v_rs < kMaxFusedRowStride);
     const bool split = rows == kSplitRows;
     const int64_t n_qt = (a.seq + rows - 1) / rows;
     const int64_t total = n_qt * a.heads * a.batch;
@@ -235,7 +241,7 @@ hipError_t launch_dp(const AttnLaunch &a, hipStream_t stream) {
         p.rot_units = (int)(n_qt / (kXcds << shift));
         p.by_rot = make_fastdiv((uint32_t)(p.rot_units << shift));
     }
-    if constexpr (FUSED) {
+    if constexpr (PARTS) {
         if (rows == kPartRows) return launch_parts(a, p, stream);
     }
     const dim3 grid((unsigned)total), block(kThreads);

@@ -1193,6 +1193,7 @@ __device__ __forceinline__ void attend_body(const AttnLaunch &a, const Plan &p, 
                 if (ragged && !zero_row && !finite4(y))
                     y = exact_chunk(a.q + base(a.q_bs, a.q_hs, a.q_rs) + (int64_t)qi * a.q_rs, kb, a.k_rs, vb,
                                     a.v_rs, rr.lo, rr.hi, D, a.scale, g * DQ + 4 * c);
+                if (REDO && finite4(*(const float4 *)(orow + 4 * c))) continue;
                 *(float4 *)(orow + 4 * c) = y;
             }
         }
@@ -1223,7 +1224,7 @@ constexpr int64_t kMaxFusedRowStride = (int64_t(1) << 31) / (4 * kKeys) - kKeys;
 
 constexpr int kPartRows = 128;  // query rows of an attention_parts.hip item
 
-// attention_parts.hip: Full, Block3 and Sliding at head_dim 64, one workgroup per 128 query rows
+// attention_parts.hip: Full, Block3 and Sliding at head_dim 64 or 128, one workgroup per 128 query rows
 // (plan: n_qt of them per (sequence, head)).
 hipError_t launch_parts(const AttnLaunch &a, const Plan &p, hipStream_t stream);
 

@@ -1,4 +1,4 @@
-// Attention at head_dim 64 on three-part bfloat16 products: 128 query rows per workgroup.
+// Attention at head_dim 64 and 128 on three-part bfloat16 products: 128 query rows per workgroup.
 //
 // The fp32 matrix instruction bounds the multi-tile masks (Block3 at 16 x 8192 rows ran at
 // 113 of its 155 TFLOP/s).  Here every operand of both products is the exact sum of three
@@ -6,13 +6,14 @@
 // 6 / 16 of the fp32 instruction's time, fewer roundings, and the probabilities keep all their
 // 24 bits.  Splitting costs 5.5 VALU operations an element, so a workgroup takes 128 rows:
 // each K and V element is split once for all of them, and each wave's 32 rows fill the
-// 32 x 32 x 16 instruction.  A wave's tile of 64 keys is 96 matrix instructions (3,072 clocks)
+// 32 x 32 x 16 instruction.  At head_dim 64 a wave's tile of 64 keys is 96 matrix instructions (3,072 clocks)
 // and about 500 VALU operations (2,400 at the 4.7 clocks they sustain); two waves a SIMD overlap
 // them to about 3,900 clocks a tile.
 //
 // Measured (us, before on the 64-row fp32 kernel): Block3 16 x 8192 116 -> 77 (165 TFLOP/s),
 // Block3 32 x 12 x 2048 402 -> 300, Full 4 x 12 x 2048 (1024 to 2048 valid) 342 -> 219, Full
-// 1 x 12 x 4096 442 -> 294 (175 TFLOP/s); relative 2-norm error against float64 4.6e-7 -> 3.9e-7
+// 1 x 12 x 4096 442 -> 294 (175 TFLOP/s); head_dim 128: Block3 8 x 8 x 2048 228 -> 167, Full
+// 2 x 8 x 2048 290 -> 185 (186 TFLOP/s); relative 2-norm error against float64 4.6e-7 -> 3.9e-7
 // (Block3), 7.7e-7 -> 7.0e-7 (Full).
 //
 //   S^T = K Q^T (32 keys x 32 queries per subtile), online softmax as in attention_body.hpp,
@@ -39,14 +40,15 @@ namespace raya {
 namespace attn {
 namespace {
 
-// acc[i] += a[i] b over the parts, the smallest products first; the two sums alternate, so that
+// acc[i] += a[i] b over the parts, the smallest products first; the sums alternate, so that
 // no instruction waits for the one before it.
-__device__ __forceinline__ void products(const bf16x8 (&a)[2][3], const bf16x8 (&b)[3], floatx16 (&acc)[2]) {
+template <int N>
+__device__ __forceinline__ void products(const bf16x8 (&a)[N][3], const bf16x8 (&b)[3], floatx16 (&acc)[N]) {
     constexpr int qa[6] = {2, 0, 1, 1, 0, 0}, qb[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
     for (int q = 0; q < 6; ++q)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i] = mfma_bf16(a[i][qa[q]], b[qb[q]], acc[i]);
+        for (int i = 0; i < N; ++i) acc[i] = mfma_bf16(a[i][qa[q]], b[qb[q]], acc[i]);
 }
 __device__ __forceinline__ void product(const bf16x8 (&a)[3], const bf16x8 (&b)[3], floatx16 &acc) {
     constexpr int qa[6] = {2, 0, 1, 1, 0, 0}, qb[6] = {0, 2, 1, 0, 1, 0};
@@ -54,14 +56,17 @@ __device__ __forceinline__ void product(const bf16x8 (&a)[3], const bf16x8 (&b)[
     for (int q = 0; q < 6; ++q) acc = mfma_bf16(a[qa[q]], b[qb[q]], acc);
 }
 
-constexpr int D = 64, DS = D / 16, DT = D / 32;  // head_dim, its MFMA steps and 32-wide tiles
-constexpr int kPlane = kKeys * D * 2;            // bytes of one part of a K or V tile
-constexpr int kPartTile = 3 * kPlane;
+// Bytes of one part of a K or V tile, and of a tile.
+template <int D>
+constexpr int kPlane = kKeys * D * 2;
+template <int D>
+constexpr int kPartTile = 3 * kPlane<D>;
 
 // K part blocks: [32-key subtile][step][h][32 keys][8 dims]; key row r of the block at slot
-// r ^ (2 step + h), so that the 16 lanes that write one row's chunks cover 128 bytes.
+// r ^ ((2 step + h) mod 8), so that the 16 lanes that write one row's chunks cover 128 bytes.
+template <int D>
 __device__ __forceinline__ int k_slot(int key, int step, int h) {
-    return ((key >> 5) * DS + step) * 1024 + h * 512 + ((key & 31) ^ (2 * step + h)) * 16;
+    return ((key >> 5) * (D / 16) + step) * 1024 + h * 512 + ((key & 31) ^ ((2 * step + h) & 7)) * 16;
 }
 // V part blocks: [32-dim tile][16-key step][h][32 dims][8 keys]; dim row d at slot
 // d ^ ((d / 4) & 7), so that 8 lanes writing dims 4 apart hit 8 different slots mod 8.
@@ -88,8 +93,10 @@ __device__ __forceinline__ Item decode_longest_first(const AttnLaunch &a, const 
     return decode<kPartRows, RAYA_MASK_FULL>(a, p, item + (seq - slot) * a.heads * p.n_qt);
 }
 
-template <int MK, bool TIMED>
+template <int D, int MK, bool TIMED>
 __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, char *lds, StageClock *clk) {
+    constexpr int DS = D / 16, DT = D / 32, CH = D / 4;  // MFMA steps, 32-wide tiles and 16-byte chunks of a row
+    constexpr int PLANE = kPlane<D>;
     // Windows leave each wave whole subtiles outside its rows' keys; the block masks' items see
     // every key of their range.
     constexpr bool WINDOW = MK == RAYA_MASK_SLIDING;
@@ -106,9 +113,9 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
     float *ob = a.out + base(a.o_bs, a.o_hs, a.o_rs);
     if (it.k_lo >= it.k_hi) {  // every row is padding: write zeros
         if (packed) return;
-        for (int c = tid; c < kPartRows * 16; c += kThreads) {
-            const int r = it.q0 + c / 16;
-            if (r < a.seq) store_stream(ob + (int64_t)r * a.o_rs + 4 * (c % 16), make_float4(0.f, 0.f, 0.f, 0.f));
+        for (int c = tid; c < kPartRows * CH; c += kThreads) {
+            const int r = it.q0 + c / CH;
+            if (r < a.seq) store_stream(ob + (int64_t)r * a.o_rs + 4 * (c % CH), make_float4(0.f, 0.f, 0.f, 0.f));
         }
         return;
     }
@@ -132,49 +139,51 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
         return it.k_lo + (j >= n_tiles ? j - n_tiles : j) * kKeys;
     };
 
-    // Staging.  K: 16 lanes take a row's 16-byte chunks, 16 rows a pass.  V: each thread takes 4
-    // keys x 4 dims (key quad 4 s + 2 half + vh of PV step s), so that it can write 4 keys of a
-    // dim together.
-    const int kc = tid & 15, kr = tid >> 4;
+    // Staging.  K: CH lanes take a row's 16-byte chunks.  V: each thread takes 4 keys x 4 dims
+    // (key quad 4 s + 2 half + vh of PV step s), for every 64 dims, so that it can write 4 keys
+    // of a dim together.
+    constexpr int KR = kThreads / CH, PUTS = kKeys / KR;  // rows a pass and passes; V: PUTS dims a thread
+    const int kc = tid % CH, kr = tid / CH;
     const int vs = wave, half = (lane >> 3) & 1, vh = (lane >> 4) & 1, dq = (lane & 7) + 8 * (lane >> 5);
     const int vkey = 16 * vs + 8 * half + 4 * vh;
-    float4 kreg[4], vreg[4];
-    // Keys past the item's last one are fetched as copies of it.
+    float4 kreg[PUTS], vreg[PUTS];
+    // Keys past the item's last one are fetched as copies of it (they weigh 0), tiles past the
+    // last one as copies of that (a branch would make the registers in flight wait).
     const auto load_k = [&](int j) {
         const int kt = tile_at(min(j, n_tiles - 1)), last = it.k_hi - 1 - kt;
         const float *src = kb + (int64_t)kt * a.k_rs;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            kreg[i] = *(const float4 *)(src + (uint32_t)(min(kr + 16 * i, last) * (int)a.k_rs) + 4 * kc);
+        for (int i = 0; i < PUTS; ++i)
+            kreg[i] = *(const float4 *)(src + (uint32_t)(min(kr + KR * i, last) * (int)a.k_rs) + 4 * kc);
     };
     const auto load_v = [&](int j) {
         const int kt = tile_at(min(j, n_tiles - 1)), last = it.k_hi - 1 - kt;
         const float *src = vb + (int64_t)kt * a.v_rs;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-            vreg[i] = *(const float4 *)(src + (uint32_t)(min(vkey + i, last) * (int)a.v_rs) + 4 * dq);
+        for (int i = 0; i < PUTS; ++i)
+            vreg[i] = *(const float4 *)(src + (uint32_t)(min(vkey + i % 4, last) * (int)a.v_rs) + 64 * (i / 4) + 4 * dq);
     };
-    char *kl = lds, *vl = lds + kPartTile;
+    char *kl = lds, *vl = lds + kPartTile<D>;
     const auto put_k = [&](int i) {
         uint32_t lo[3], hi[3];
         split3(kreg[i].x, kreg[i].y, lo);
         split3(kreg[i].z, kreg[i].w, hi);
-        char *d = kl + k_slot(kr + 16 * i, kc >> 2, (kc >> 1) & 1) + (kc & 1) * 8;
+        char *d = kl + k_slot<D>(kr + KR * i, kc >> 2, (kc >> 1) & 1) + (kc & 1) * 8;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * kPlane) = uint32x2{lo[q], hi[q]};
+        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * PLANE) = uint32x2{lo[q], hi[q]};
     };
-    // Dim 4 dq + i of this thread's four keys.
+    // Dim 64 (i / 4) + 4 dq + i % 4 of this thread's four keys.
     const auto put_v = [&](int i) {
         const auto at = [&](int k) {
-            const float4 &x = vreg[k];
-            return i == 0 ? x.x : i == 1 ? x.y : i == 2 ? x.z : x.w;
+            const float4 &x = vreg[i / 4 * 4 + k];
+            return i % 4 == 0 ? x.x : i % 4 == 1 ? x.y : i % 4 == 2 ? x.z : x.w;
         };
         uint32_t lo[3], hi[3];
         split3(at(0), at(1), lo);
         split3(at(2), at(3), hi);
-        char *d = vl + v_slot(4 * dq + i, vs, vh) + half * 8;
+        char *d = vl + v_slot(64 * (i / 4) + 4 * dq + i % 4, vs, vh) + half * 8;
 #pragma unroll
-        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * kPlane) = uint32x2{lo[q], hi[q]};
+        for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * PLANE) = uint32x2{lo[q], hi[q]};
     };
 
     load_k(0);
@@ -201,7 +210,7 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
         }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) put_k(i);
+    for (int i = 0; i < PUTS; ++i) put_k(i);
     load_k(1);
     __syncthreads();
 
@@ -240,12 +249,12 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
                         bf16x8 kf[3];
 #pragma unroll
                         for (int q = 0; q < 3; ++q)
-                            kf[q] = *(const bf16x8 *)(kl + q * kPlane + k_slot(32 * t + li, d, h));
+                            kf[q] = *(const bf16x8 *)(kl + q * PLANE + k_slot<D>(32 * t + li, d, h));
                         product(kf, qf[d], s[t]);
                     }
                 }
-                put_v(2 * t);
-                put_v(2 * t + 1);
+#pragma unroll
+                for (int i = t * PUTS / 2; i < (t + 1) * PUTS / 2; ++i) put_v(i);
             }
         } else {
 #pragma unroll
@@ -255,9 +264,9 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
                 for (int t = 0; t < 2; ++t)
 #pragma unroll
                     for (int q = 0; q < 3; ++q)
-                        kf[t][q] = *(const bf16x8 *)(kl + q * kPlane + k_slot(32 * t + li, d, h));
+                        kf[t][q] = *(const bf16x8 *)(kl + q * PLANE + k_slot<D>(32 * t + li, d, h));
                 products(kf, qf[d], s);
-                put_v(d);
+                put_v(d);  // PUTS = DS
             }
         }
         load_v(j + 1);
@@ -331,17 +340,17 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
                     for (int d = 0; d < DT; ++d)
 #pragma unroll
                         for (int q = 0; q < 3; ++q)
-                            vf[d][q] = *(const bf16x8 *)(vl + q * kPlane + v_slot(32 * d + li, 2 * t + u, h));
+                            vf[d][q] = *(const bf16x8 *)(vl + q * PLANE + v_slot(32 * d + li, 2 * t + u, h));
                     products(vf, pf, oacc);
                 }
             }
-            put_k(2 * t);
-            put_k(2 * t + 1);
+#pragma unroll
+            for (int i = t * PUTS / 2; i < (t + 1) * PUTS / 2; ++i) put_k(i);
         }
         load_k(j + 2);
         if constexpr (TIMED) {
             settle(oacc[0][15]);
-            settle(oacc[1][15]);
+            settle(oacc[DT - 1][15]);
             lap(clk, clk->pv);
         }
         __syncthreads();
@@ -368,8 +377,8 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
         }
     const int rows = packed ? valid : a.seq;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane >> 4), c = lane & 15;
+    for (int i = 0; i < CH / 2; ++i) {
+        const int at = i * 64 + lane, r = at / CH, c = at % CH;
         const float4 y = *(const float4 *)(st + r * D + 4 * (c ^ (r & 15)));
         if (qw + r < rows) store_stream(ob + (int64_t)(qw + r) * a.o_rs + 4 * c, y);
     }
@@ -382,48 +391,59 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
             half_item.q0 = q0;
             half_item.k_lo = key_range(MK, arg, p.by_arg, q0, valid).lo;
             half_item.k_hi = key_range(MK, arg, p.by_arg, min(q0 + kQRows, valid) - 1, valid).hi;
-            attend_body<D, true, false, WINDOW, false, MK, false, 0, WINDOW, true>(a, p, half_item, (float *)lds,
+            attend_body<D, D == 64, false, WINDOW && D == 64, false, MK, false, 0, WINDOW, true>(a, p, half_item, (float *)lds,
                                                                                   (float *)lds + kKeys * D, nullptr);
             __syncthreads();
         }
     }
 }
 
-template <int MK>
-__global__ void __launch_bounds__(kThreads, 2) attend_parts_kernel(const AttnLaunch a, const Plan p) {
-    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile];
-    parts_body<MK, false>(a, p, lds, nullptr);
+// Waves per SIMD: at head_dim 128 Q's parts and the output take 160 registers by themselves.
+template <int D>
+constexpr int kPartWaves = D == 64 ? 2 : 1;
+
+template <int D, int MK>
+__global__ void __launch_bounds__(kThreads, kPartWaves<D>) attend_parts_kernel(const AttnLaunch a, const Plan p) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile<D>];
+    parts_body<D, MK, false>(a, p, lds, nullptr);
 }
 
 // The same with the stage clock (attention.hip's attend_timed_kernel).
-template <int MK>
-__global__ void __launch_bounds__(kThreads, 2) attend_parts_timed_kernel(const AttnLaunch a, const Plan p) {
-    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile];
+template <int D, int MK>
+__global__ void __launch_bounds__(kThreads, kPartWaves<D>) attend_parts_timed_kernel(const AttnLaunch a, const Plan p) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * kPartTile<D>];
     __shared__ uint64_t part[kWaves][5];
     StageClock c{};
-    parts_body<MK, true>(a, p, lds, &c);
+    parts_body<D, MK, true>(a, p, lds, &c);
     add_stage_totals(a, c, part);
 }
 
-template <int MK>
-void launch_mask(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
+template <int D, int MK>
+hipError_t launch_mask(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
     const dim3 grid((unsigned)p.total), block(kThreads);
     if (a.stage_cycles)
-        hipLaunchKernelGGL((attend_parts_timed_kernel<MK>), grid, block, 0, stream, a, p);
+        hipLaunchKernelGGL((attend_parts_timed_kernel<D, MK>), grid, block, 0, stream, a, p);
     else
-        hipLaunchKernelGGL((attend_parts_kernel<MK>), grid, block, 0, stream, a, p);
+        hipLaunchKernelGGL((attend_parts_kernel<D, MK>), grid, block, 0, stream, a, p);
+    return hipGetLastError();
+}
+
+template <int D>
+hipError_t launch_dim(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
+    switch (a.mask_kind) {
+    case RAYA_MASK_BLOCK3: return launch_mask<D, RAYA_MASK_BLOCK3>(a, p, stream);
+    case RAYA_MASK_FULL: return launch_mask<D, RAYA_MASK_FULL>(a, p, stream);
+    case RAYA_MASK_SLIDING: return launch_mask<D, RAYA_MASK_SLIDING>(a, p, stream);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace
 
 hipError_t launch_parts(const AttnLaunch &a, const Plan &p, hipStream_t stream) {
-    switch (a.mask_kind) {
-    case RAYA_MASK_BLOCK3: launch_mask<RAYA_MASK_BLOCK3>(a, p, stream); break;
-    case RAYA_MASK_FULL: launch_mask<RAYA_MASK_FULL>(a, p, stream); break;
-    case RAYA_MASK_SLIDING: launch_mask<RAYA_MASK_SLIDING>(a, p, stream); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    if (a.head_dim == 64) return launch_dim<64>(a, p, stream);
+    if (a.head_dim == 128) return launch_dim<128>(a, p, stream);
+    return hipErrorInvalidValue;
 }
 
 }  // namespace attn

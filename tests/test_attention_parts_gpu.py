@@ -1,4 +1,4 @@
-"""The 128-row attention kernel on three-part bfloat16 products, forced with RAYA_ATTN_ITEMS=128:
+"""The 128-row attention kernel (head_dim 64 and 128) on three-part bfloat16 products, forced with RAYA_ATTN_ITEMS=128:
 edges of its tiles and waves under every mask it takes, strided and padded batches, non-finite
 operands, and its instrumented copy.
 
@@ -44,15 +44,17 @@ def close(got, want):
 
 @pytest.mark.parametrize("name", list(MASKS))
 @pytest.mark.parametrize("seq", [1, 31, 33, 64, 127, 129, 300, 513])
-def test_edges(hip_attention, name, seq):
+@pytest.mark.parametrize("d", [64, 128])
+def test_edges(hip_attention, name, seq, d):
     """One launch of sequences whose valid lengths end at, before and after every kind of edge."""
     h = 2
     lens = sorted({max(0, min(seq, n)) for n in (0, 1, 16, 32, 65, 128, 130, 257, seq - 1, seq)})
-    qkv = [inputs(100 + n, h, seq) for n in range(len(lens))]
+    qkv = [inputs(100 + n, h, seq, d) for n in range(len(lens))]
     dev = [torch.from_numpy(np.stack([x[i] for x in qkv])).cuda() for i in range(3)]
     out = torch.full_like(dev[0], 7.0)
     print(f"{name} seq {seq} lens {lens}", flush=True)
-    hip_attention.attend_batched(*dev, out, torch.tensor(lens, dtype=torch.int32, device="cuda"), MASKS[name][0])
+    hip_attention.attend_batched(*dev, out, torch.tensor(lens, dtype=torch.int32, device="cuda"), MASKS[name][0],
+                                 0.125)
     got = out.cpu().numpy()
     for b, n in enumerate(lens):
         assert (got[b, :, n:] == 0).all()
@@ -85,17 +87,18 @@ def test_packed_projection_and_scales(hip_attention, name, scale):
 
 @pytest.mark.parametrize("name", list(MASKS))
 @pytest.mark.parametrize("operand", [0, 1, 2])
-def test_non_finite_operands_match_the_reference(hip_attention, name, operand):
+@pytest.mark.parametrize("d", [64, 128])
+def test_non_finite_operands_match_the_reference(hip_attention, name, operand, d):
     """Inf, -Inf, NaN and 3.4e38 in one row of q, k or v at a time: NaN and Inf where Naive has
     them, its values elsewhere."""
     h, s, valid = 1, 300, 290
     for at, value in ((0, np.inf), (63, -np.inf), (130, np.nan), (valid - 1, -np.inf), (200, 3.4e38)):
-        x = inputs(9, h, s)
+        x = inputs(9, h, s, d)
         x[operand][0, at, 5] = value
         with np.errstate(all="ignore"):
             want = naive(*x, name, valid)
-        out = np.full(h * s * 64, 7.0, np.float32)
-        hip_attention.attend(R.AttnShape(h, s, 64), R.AttnParams(MASKS[name][0], 128, valid, 0.125),
+        out = np.full(h * s * d, 7.0, np.float32)
+        hip_attention.attend(R.AttnShape(h, s, d), R.AttnParams(MASKS[name][0], 128, valid, 0.125),
                              *(t.reshape(-1) for t in x), out)
         got = out.reshape(want.shape)
         assert np.array_equal(np.isnan(got), np.isnan(want)), (at, value)
@@ -105,17 +108,18 @@ def test_non_finite_operands_match_the_reference(hip_attention, name, operand):
 
 
 @pytest.mark.parametrize("name", ["block3", "full", "sliding64"])
-def test_error_is_no_larger_than_the_fp32_kernels(hip_attention, monkeypatch, name):
+@pytest.mark.parametrize("d", [64, 128])
+def test_error_is_no_larger_than_the_fp32_kernels(hip_attention, monkeypatch, name, d):
     """RMS distance from float64 attention, against the 64-row kernel's on the fp32 instruction."""
     h, s = 4, 1024
-    x = inputs(5, h, s)
+    x = inputs(5, h, s, d)
     dev = [torch.from_numpy(t[None]).cuda() for t in x]
     valid = torch.tensor([s], dtype=torch.int32, device="cuda")
     outs = {}
     for items in ("128", "64"):
         monkeypatch.setenv("RAYA_ATTN_ITEMS", items)
         outs[items] = torch.empty_like(dev[0])
-        hip_attention.attend_batched(*dev, outs[items], valid, MASKS[name][0])
+        hip_attention.attend_batched(*dev, outs[items], valid, MASKS[name][0], 0.125)
     q, k, v = (t[0].double() for t in dev)
     i = torch.arange(s, device="cuda")
     seen = {"block3": (i[:, None] // 128 - i[None] // 128).abs() <= 1, "full": (i[:, None] >= 0) & (i[None] >= 0),
@@ -128,11 +132,12 @@ def test_error_is_no_larger_than_the_fp32_kernels(hip_attention, monkeypatch, na
 
 
 @pytest.mark.parametrize("name", ["block3", "sliding64"])
-def test_stages(hip_attention, name):
+@pytest.mark.parametrize("d", [64, 128])
+def test_stages(hip_attention, name, d):
     """The instrumented copy: the same outputs, the tiles of 16 rows x 64 keys it computes (two to
     a wave of 32 rows that meets the tile, one if its second 16 are padding)."""
     seq, heads, lens = 512, 2, [512, 300]
-    dev = [torch.from_numpy(np.stack([inputs(n, heads, seq)[i] for n in (1, 2)])).cuda() for i in range(3)]
+    dev = [torch.from_numpy(np.stack([inputs(n, heads, seq, d)[i] for n in (1, 2)])).cuda() for i in range(3)]
     valid = torch.tensor(lens, dtype=torch.int32, device="cuda")
     mask = MASKS[name][0]
     plain = torch.empty_like(dev[0])
