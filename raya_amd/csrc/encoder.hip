@@ -10,6 +10,7 @@
 #include <cmath>
 
 #include "internal.hpp"
+#include "row_norm.hpp"
 
 namespace raya {
 namespace {
@@ -211,28 +212,17 @@ unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per)
 
 namespace {
 
-// The pre-LN LayerNorm statistics of each row from its 64-column chunks'
-// (c, r = sum (x - c), s = sum (x - c)^2), in f64 as ops::layer_norm keeps its
-// statistics (crates/raya-core/src/ops.rs:51-74): a chunk's mean is c + r / 64 and
-// its sum of squared deviations s - r^2 / 64; the chunks combine as Chan et al.'s
-// pairwise update.  Out: (mean_hi, mean_lo, 1 / sqrt(var + eps), 0) with var the
-// biased variance and mean_hi + mean_lo the f64 mean to 48 bits.
 __global__ void ln_stats_kernel(const float4 *chunks_in, int rows, int chunks, float eps, float4 *out) {
     const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= rows) return;
-    const float4 *st = chunks_in + (int64_t)row * chunks;
-    double mean = 0.0;
-    for (int c = 0; c < chunks; ++c) mean += (double)st[c].x + (double)st[c].y * (1.0 / 64.0);
-    mean /= chunks;
-    double m2 = 0.0;
-    for (int c = 0; c < chunks; ++c) {
-        const double r = st[c].y, cm = (double)st[c].x + r * (1.0 / 64.0);
-        const double dm = cm - mean;
-        m2 += ((double)st[c].z - r * r * (1.0 / 64.0)) + 64.0 * dm * dm;
-    }
-    const double var = fmax(m2, 0.0) / (64.0 * chunks);
-    const float hi = (float)mean;
-    out[row] = make_float4(hi, (float)(mean - (double)hi), (float)(1.0 / sqrt(var + (double)eps)), 0.0f);
+    if (row < rows) out[row] = row_norm(chunks_in + (int64_t)row * chunks, chunks, eps);
+}
+
+// out = b with `gain` multiplied into its columns, each product rounded to f32.
+__global__ void fold_gain_kernel(const float4 *b, const float4 *gain, int64_t n4, int k4, float4 *out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n4) return;
+    const float4 x = b[i], g = gain[i % k4];
+    out[i] = make_float4(__fmul_rn(x.x, g.x), __fmul_rn(x.y, g.y), __fmul_rn(x.z, g.z), __fmul_rn(x.w, g.w));
 }
 
 // One wave per row: each lane sums a strided share of the row in f64, then the
@@ -253,6 +243,14 @@ __global__ void row_sums_kernel(const float *b, int64_t ldb, int rows, int k, fl
 hipError_t launch_row_sums(const float *b, int64_t ldb, int rows, int k, float *sums, hipStream_t stream) {
     if (rows <= 0) return hipSuccess;
     hipLaunchKernelGGL(row_sums_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, b, ldb, rows, k, sums);
+    return hipGetLastError();
+}
+
+hipError_t launch_fold_gain(const float *b, const float *gain, int rows, int k, float *out, hipStream_t stream) {
+    if (rows <= 0 || k % 4 != 0) return hipErrorInvalidValue;
+    const int64_t n4 = (int64_t)rows * (k / 4);
+    hipLaunchKernelGGL(fold_gain_kernel, dim3(blocks_for(n4, 256)), dim3(256), 0, stream, (const float4 *)b,
+                       (const float4 *)gain, n4, k / 4, (float4 *)out);
     return hipGetLastError();
 }
 

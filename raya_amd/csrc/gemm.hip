@@ -68,18 +68,19 @@ GemmPlan plan_of(int m, int n, int k, int act, bool vec, bool whole, size_t room
 hipError_t launch(const GemmLaunch &g, hipStream_t stream) {
     constexpr int kNone = RAYA_EPI_NONE, kGeglu = RAYA_EPI_GEGLU;
     const int act = g.act;
-    if (g.in_stats || g.out_stats) {
+    const bool norm = g.in_stats || g.in_chunks;
+    if (norm || g.out_stats) {
         // Only the staged epilogue carries them (see GemmLaunch).
         const bool vec_out = (g.ldo & 3) == 0 && ((uintptr_t)g.out & 15) == 0 &&
                              (!g.residual || ((g.ldr & 3) == 0 && ((uintptr_t)g.residual & 15) == 0));
         if (!vec_out) return hipErrorInvalidValue;
-        if (g.in_stats && !g.colsum) return hipErrorInvalidValue;
+        if (norm && (!g.colsum || (!g.in_stats && g.k % 64 != 0))) return hipErrorInvalidValue;
         if (g.out_stats && (act != kNone || g.n % 64 != 0)) return hipErrorInvalidValue;
     }
     if (g.rope_cos && (act != kNone || g.rope_cols % kRopeHeadDim != 0 || g.rope_cols > g.n))
         return hipErrorInvalidValue;
     if (g.reduce || g.splits > 1) return hipErrorInvalidValue;  // launch_gemm's own fields
-    const GemmPlan p = plan_of(g.m, g.n, g.k, act, aligned_rows(g), g.in_stats || g.out_stats,
+    const GemmPlan p = plan_of(g.m, g.n, g.k, act, aligned_rows(g), norm || g.out_stats,
                                g.partials ? g.partial_floats : 0);
     const int64_t tiles = tiles_of(p.tile, g.m, g.n, act);
     if (tiles * p.splits > 0x7fffffff / 512) return hipErrorInvalidValue;

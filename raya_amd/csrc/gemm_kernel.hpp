@@ -46,6 +46,7 @@
 
 #include "internal.hpp"
 #include "parts.hpp"
+#include "row_norm.hpp"
 
 namespace raya {
 namespace gemm {
@@ -316,10 +317,11 @@ struct Tile {
     static constexpr int PLANE = ROWS * BK * 2;   // bytes of one part of a slab
     static constexpr int STAGE = 3 * PLANE;
     // After the K loop the ring holds the other groups' sums, then each wave's epilogue
-    // staging, then the input rows' norms.
+    // staging.
     static constexpr int SUMS = (WK - 1) * GROUP * TM * 32 * 64 * 4;
     static constexpr int STAGING = SUMS + GROUP * kStageFloats * 4;
-    static constexpr int LDS = std::max(2 * STAGE, STAGING + BM * 8);
+    static constexpr int NORMS = std::max(2 * STAGE, STAGING);  // the input rows' norms, past both
+    static constexpr int LDS = NORMS + BM * 16;
     static_assert(KS % WK == 0, "every group takes whole MFMA steps of a slab");
 };
 
@@ -392,6 +394,17 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
     const int wm = wg / T::WN * 32 * TM, wn = wg % T::WN * 64;
     const int li = lane & 31, h = lane >> 5;
 
+    // The input rows' (mean_hi, mean_lo, rstd), one row per thread.
+    float4 *norms = (float4 *)(ring + T::NORMS);
+    if constexpr (NORM) {
+        static_assert(T::BM <= T::THREADS, "a thread per row");
+        if (tid < T::BM) {
+            const int row = min(m0 + tid, g.m - 1), chunks = g.k / 64;
+            norms[tid] = g.in_stats ? g.in_stats[row] : row_norm(g.in_chunks + (int64_t)row * chunks, chunks, g.in_eps);
+        }
+        __syncthreads();
+    }
+
     floatx16 acc[TM][2];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -433,7 +446,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
                 const int row = min(m0 + r0 + p * RPP, g.m - 1);
                 src[p] = g.a + (int64_t)row * g.lda + 4 * c;
                 cen[p] = 0.f;
-                if constexpr (NORM) cen[p] = norm_centre(g.in_stats[row]);
+                if constexpr (NORM) cen[p] = norm_centre(norms[r0 + p * RPP]);
             } else {
                 src[p] = g.b + (int64_t)b_row<GEGLU>(g, n0, r0 + p * RPP - T::BM) * g.ldb + 4 * c;
             }
@@ -573,15 +586,6 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
             return;
         }
     }
-    // The input rows' (rest, rstd), one row per thread.
-    float2 *rownorm = (float2 *)(ring + T::STAGING);
-    if constexpr (NORM) {
-        for (int r = tid; r < T::BM; r += T::THREADS) {
-            const float4 st = g.in_stats[min(m0 + r, g.m - 1)];
-            rownorm[r] = make_float2((st.x - norm_centre(st)) + st.y, st.z);
-        }
-        __syncthreads();
-    }
     if (group > 0) return;
 
     // From here on single floats: a 16-register vector changed in a branch would be held twice.
@@ -602,7 +606,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
             if (__any(bad)) {
                 const int row = min(m0 + wm + 32 * i + li, g.m - 1);
                 float cen = 0.f;
-                if constexpr (NORM) cen = norm_centre(g.in_stats[row]);
+                if constexpr (NORM) cen = norm_centre(norms[wm + 32 * i + li]);
                 const floatx16 e =
                     exact_subtile(g.a + (int64_t)row * g.lda,
                                   g.b + (int64_t)b_row<GEGLU>(g, n0, wn + 32 * j + li) * g.ldb, g.k, h, cen);
@@ -629,9 +633,10 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
             if constexpr (NORM) {
                 // rstd (y - rest colsum), rest = (mean_hi - centre) + mean_lo the part of the
                 // mean that the centring left (norm_centre).
-                const float2 st = rownorm[wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3)];
+                const float4 st = norms[wm + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3)];
+                const float rest = (st.x - norm_centre(st)) + st.y;
 #pragma unroll
-                for (int j = 0; j < 2; ++j) y[i][j][r] = st.y * (y[i][j][r] - st.x * cs[j]);
+                for (int j = 0; j < 2; ++j) y[i][j][r] = st.z * (y[i][j][r] - rest * cs[j]);
             }
             // Without a bias the sum is used as it is (x + 0 would turn -0 into +0).
 #pragma unroll
@@ -664,7 +669,7 @@ template <class T, bool GEGLU>
 hipError_t launch_tile(const GemmLaunch &g, unsigned grid, hipStream_t stream) {
     const dim3 blocks(grid), threads(T::THREADS);
     const bool vec = aligned_rows(g), pad = !vec || g.k % T::BK != 0;
-    if (g.in_stats) {  // folded LayerNorm: QKV (with or without RoPE) and GeGLU
+    if (g.in_stats || g.in_chunks) {  // folded LayerNorm: QKV (with or without RoPE) and GeGLU
         if (pad) return hipErrorInvalidValue;
         hipLaunchKernelGGL((gemm_kernel<T, GEGLU, true, false, 0>), blocks, threads, 0, stream, g);
     } else if (g.out_stats) {  // the residual GEMMs

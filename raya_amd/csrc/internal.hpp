@@ -68,8 +68,13 @@ struct GemmLaunch {
     // ops::layer_norm removes it before scaling; the rest of the mean comes out
     // as mean colsum.  Then y = rstd (acc - mean' colsum) before bias, activation
     // and RoPE: LayerNorm(a) W^T.  Null: off.
+    // Or, with in_stats null, in_chunks: the rows' chunk statistics as out_stats writes them
+    // ([m][k / 64]; in_eps the norm's), which each workgroup combines for its own rows as
+    // launch_ln_stats would.
     const float4 *in_stats;
     const float *colsum;
+    const float4 *in_chunks;
+    float in_eps;
     // Per output row and 64-column chunk, after the residual add ([m][n / 64]; n a
     // multiple of 64): (c, sum (x - c), sum (x - c)^2, 0) with c the chunk's f32
     // mean, the same c in every lane, so that launch_ln_stats recovers the chunk's
@@ -115,6 +120,8 @@ hipError_t launch_layer_norm(const LayerNormLaunch &l, hipStream_t stream);
 // Each row's (mean_hi, mean_lo, 1 / sqrt(var + eps), 0) from its 64-column chunk
 // statistics (GemmLaunch::out_stats, [rows][n_chunks]) into out ([rows]).
 hipError_t launch_ln_stats(const float4 *chunks, int rows, int n_chunks, float eps, float4 *out, hipStream_t stream);
+// out = b ([rows][k], k a multiple of 4, 16-byte aligned) with `gain` ([k]) multiplied into its columns.
+hipError_t launch_fold_gain(const float *b, const float *gain, int rows, int k, float *out, hipStream_t stream);
 // sums[j] = sum over t < k of b[j][t] in f64, rounded to f32 ([rows]).
 hipError_t launch_row_sums(const float *b, int64_t ldb, int rows, int k, float *sums, hipStream_t stream);
 hipError_t launch_rope(float *qkv, int64_t ld, const int32_t *positions, const float *cos_t,

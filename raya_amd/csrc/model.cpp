@@ -632,66 +632,54 @@ int ensure_device(Model &m, DeviceModel **out) {
 
 // LN(x) W^T = rstd ((x - c) (g * W)^T - (mean - c) colsum) with g the norm's gain, colsum[j]
 // the row sums of g * W and c a per-row centre (0, or the mean's leading part for rows far
-// from zero; GemmLaunch::in_stats).  Built on the host once per device: the products
-// g_t W[j][t] in f32 (as LN's output times W rounds them) and their row sums in f64.  The
-// residual GEMMs that produce the statistics need whole 64-column chunks (hidden a multiple of
-// 64) and depths the kernels do not pad (multiples of 16: hidden and the MLP's intermediate
-// size); other shapes keep the LayerNorm kernels.
+// from zero; GemmLaunch::in_stats).  Built on the device once: the products g_t W[j][t] in f32
+// (as LN's output times W rounds them) and their row sums in f64.  The residual GEMMs that
+// produce the statistics need whole 64-column chunks (hidden a multiple of 64) and depths the
+// kernels do not pad (multiples of 16: hidden and the MLP's intermediate size); other shapes keep
+// the LayerNorm kernels.
 bool norms_foldable(const Config &c) { return c.hidden % 64 == 0 && c.inter % 16 == 0; }
 
-int ensure_folded(const Model &m, DeviceModel &dm) {
+int ensure_folded(const Model &m, DeviceModel &dm, hipStream_t stream) {
     const Config &c = m.cfg;
     if (!dm.folded.qkv.empty() || !norms_foldable(c)) return RAYA_OK;
     const uint64_t d = c.hidden, n3 = 3 * d, n2 = 2 * c.inter;
-    std::vector<float> host;
-    host.reserve((size_t)c.layers * (n3 + n2) * (d + 1));
-    FoldedNorms f;
-    std::vector<float> sums;
-    // Appends the folded block (rows x d) and then its row sums; blocks stay 16-byte aligned
-    // because d and every row count here are multiples of 4.
-    auto fold = [&](const std::string &w, const std::string &gain, uint64_t rows, std::vector<size_t> &off,
-                    std::vector<size_t> &off_sum) -> int {
-        const auto iw = m.w.index.find(w), ig = m.w.index.find(gain);
-        if (iw == m.w.index.end() || ig == m.w.index.end())
-            return fail(RAYA_ERR_WEIGHTS, "missing %s", (iw == m.w.index.end() ? w : gain).c_str());
-        const float *wp = m.w.host.data() + m.w.entries[iw->second].offset;
-        const float *gp = m.w.host.data() + m.w.entries[ig->second].offset;
-        off.push_back(host.size());
-        sums.assign(rows, 0.0f);
-        for (uint64_t j = 0; j < rows; ++j) {
-            double sum = 0.0;
-            for (uint64_t t = 0; t < d; ++t) {
-                const float x = wp[j * d + t] * gp[t];
-                host.push_back(x);
-                sum += x;
-            }
-            sums[j] = (float)sum;
-        }
-        off_sum.push_back(host.size());
-        host.insert(host.end(), sums.begin(), sums.end());
-        return RAYA_OK;
-    };
-    for (uint64_t i = 0; i < c.layers; ++i) {
-        const std::string p = "encoder.layers." + std::to_string(i);
-        int rc = RAYA_OK;
-        if (i > 0) {
-            rc = fold(p + ".attn.Wqkv.weight", p + ".attn_norm.weight", n3, f.qkv, f.qkv_sum);
-        } else {  // layer 0 has no attn_norm
-            f.qkv.push_back(0);
-            f.qkv_sum.push_back(0);
-        }
-        if (!rc) rc = fold(p + ".mlp.Wi.weight", p + ".mlp_norm.weight", n2, f.wi, f.wi_sum);
-        if (rc) return rc;
-    }
-    // Empty offsets mean "not built": they are set only once the upload has succeeded.
-    int rc = dm.folded.buf.reserve(host.size() * sizeof(float));
+    // Each folded block (rows x d) and then its row sums; blocks stay 16-byte aligned because d
+    // and every row count here are multiples of 4.  Layer 0 has no attn_norm.
+    int rc = dm.folded.buf.reserve(c.layers * (n3 + n2) * (d + 1) * sizeof(float));
     if (rc) return rc;
-    const hipError_t e = hipMemcpy(dm.folded.buf.ptr, host.data(), host.size() * sizeof(float), hipMemcpyHostToDevice);
-    if (e != hipSuccess) return fail_device(e, "upload folded norm weights");
-    dm.folded.qkv = std::move(f.qkv);
-    dm.folded.qkv_sum = std::move(f.qkv_sum);
-    dm.folded.wi = std::move(f.wi);
-    dm.folded.wi_sum = std::move(f.wi_sum);
+    float *const buf = (float *)dm.folded.buf.ptr;
+    std::vector<size_t> qkv, qkv_sum, wi, wi_sum;
+    size_t at = 0;
+    const auto fold = [&](const std::string &w, const std::string &gain, uint64_t rows, std::vector<size_t> &off,
+                          std::vector<size_t> &off_sum) -> int {
+        const float *wp = param(m, dm, w), *gp = param(m, dm, gain);
+        if (!wp || !gp) return fail(RAYA_ERR_WEIGHTS, "missing %s", (wp ? gain : w).c_str());
+        off.push_back(at);
+        off_sum.push_back(at + rows * d);
+        hipError_t e = launch_fold_gain(wp, gp, (int)rows, (int)d, buf + off.back(), stream);
+        if (e == hipSuccess)
+            e = launch_row_sums(buf + off.back(), (int64_t)d, (int)rows, (int)d, buf + off_sum.back(), stream);
+        at += rows * (d + 1);
+        return e == hipSuccess ? RAYA_OK : fail_device(e, "fold norm weights");
+    };
+    for (uint64_t i = 0; i < c.layers && !rc; ++i) {
+        const std::string p = "encoder.layers." + std::to_string(i);
+        if (i > 0) {
+            rc = fold(p + ".attn.Wqkv.weight", p + ".attn_norm.weight", n3, qkv, qkv_sum);
+        } else {
+            qkv.push_back(0);
+            qkv_sum.push_back(0);
+        }
+        if (!rc) rc = fold(p + ".mlp.Wi.weight", p + ".mlp_norm.weight", n2, wi, wi_sum);
+    }
+    // Later forwards may run on other streams: the offsets, empty until then, mean whole blocks.
+    const hipError_t e = hipStreamSynchronize(stream);
+    if (rc) return rc;
+    if (e != hipSuccess) return fail_device(e, "fold norm weights");
+    dm.folded.qkv = std::move(qkv);
+    dm.folded.qkv_sum = std::move(qkv_sum);
+    dm.folded.wi = std::move(wi);
+    dm.folded.wi_sum = std::move(wi_sum);
     return RAYA_OK;
 }
 
@@ -925,8 +913,8 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
     DeviceModel &dm = *dmp;
     if ((rc = ensure_rope(m, dm, (int)Lmax))) return rc;
     const bool fused = fuse_norms(c);
-    if (fused && (rc = ensure_folded(m, dm))) return rc;
     hipStream_t stream = (hipStream_t)stream_ptr;
+    if (fused && (rc = ensure_folded(m, dm, stream))) return rc;
 
     const uint64_t inter = c.inter, big = std::max(inter, c.head_ffn), nact = c.n_act;
     const uint64_t BK = B * K;
@@ -1082,6 +1070,20 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
         TRY_HIP(launch_gemm(g, stream), "gemm");
         return RAYA_OK;
     };
+    // Up to kChunkNormRows tokens the GEMMs that read h combine its rows' chunk statistics
+    // themselves, which saves a launch each time (512 tokens 1,866 -> 1,817 us, 16 tokens 1,139 ->
+    // 1,104); beyond, their workgroups' starts cost more than the launch (64 x 512 25.0 ms against
+    // 25.7, 16 x 512 7.18 against 7.22).
+    constexpr uint64_t kChunkNormRows = 2048;
+    const bool chunk_norms = T <= kChunkNormRows;
+    auto norm_rows = [&](GemmLaunch &g) {
+        if (chunk_norms) {
+            g.in_chunks = hstats;
+            g.in_eps = (float)c.norm_eps;
+        } else {
+            g.in_stats = hrow;
+        }
+    };
     // The residual GEMMs of an encoder layer: h += a W^T, and with fused norms also the
     // LayerNorm chunk statistics of the new h for the next GEMM.
     auto gemm_residual = [&](const float *a, uint64_t k, const float *wt, bool stats) -> int {
@@ -1102,7 +1104,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
         g.out_stats = stats ? hstats : nullptr;
         set_split(g);
         TRY_HIP(launch_gemm(g, stream), "residual gemm");
-        if (stats)
+        if (stats && !chunk_norms)
             TRY_HIP(launch_ln_stats(hstats, (int)T, (int)(d / 64), (float)c.norm_eps, hrow, stream), "ln stats");
         return RAYA_OK;
     };
@@ -1195,7 +1197,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
             g.n_rows_b = g.n;
             g.act = RAYA_EPI_NONE;
             if (norm_in) {
-                g.in_stats = hrow;
+                norm_rows(g);
                 g.colsum = folded + dm.folded.qkv_sum[i];
             }
             if (hd == (uint64_t)kRopeHeadDim) {
@@ -1237,7 +1239,7 @@ int raya_model_forward(raya_model *model, const raya_forward_batch *in, raya_for
             g.k = (int32_t)d;
             g.n_rows_b = (int32_t)(2 * inter);
             g.act = RAYA_EPI_GEGLU;
-            g.in_stats = hrow;
+            norm_rows(g);
             g.colsum = folded + dm.folded.wi_sum[i];
             set_split(g);
             TRY_HIP(launch_gemm(g, stream), "mlp in gemm");
