@@ -19,8 +19,8 @@ struct TileCost {
     double fixed, alone, each;
 };
 constexpr TileCost kTiles[] = {
-    {Tile256::BM, Tile256::BN, Tile256::BK, 10.0, 95.0, 120.0},
-    {Tile256x128::BM, Tile256x128::BN, Tile256x128::BK, 8.0, 40.0, 61.0},
+    {Tile256::BM, Tile256::BN, Tile256::BK, 10.0, 95.0, 118.0},
+    {Tile256x128::BM, Tile256x128::BN, Tile256x128::BK, 8.0, 40.0, 63.0},
     {Tile128::BM, Tile128::BN, Tile128::BK, 9.0, 23.0, 37.0},
     {Tile64x128::BM, Tile64x128::BN, Tile64x128::BK, 6.3, 16.0, 19.5},
     {Tile64::BM, Tile64::BN, Tile64::BK, 6.6, 9.2, 13.4},
@@ -55,7 +55,10 @@ GemmPlan plan_of(int m, int n, int k, int act, bool vec, bool whole, size_t room
         for (int s = 1; s <= 8; ++s) {
             if (s > 1 && (t == 0 || (k + c.bk - 1) / c.bk < 2 * s || partial_floats({t, s}, m, n, act) > room)) break;
             const double r = (double)(tiles * s) / kUnits;
-            const double per = r <= 1.0 ? c.alone + 0.25 * r * (c.each - c.alone) : c.each * 0.5 * (r + std::ceil(r));
+            // A last round that is not full runs faster than a full one, the less so the larger the tile.
+            const double part = t == 0 ? 0.25 : 0.5;
+            const double per = r <= 1.0 ? c.alone + 0.25 * r * (c.each - c.alone)
+                                        : c.each * (part * r + (1.0 - part) * std::ceil(r));
             double us = c.fixed + per * k / (768.0 * s);
             // The summing launch: its own fixed cost and the partials written and read once each.
             if (s > 1) us += 5.0 + partial_floats({t, s}, m, n, act) * 8.0 / 3e6;
