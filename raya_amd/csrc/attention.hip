@@ -100,31 +100,39 @@ int scatter_half_bits(int64_t total) {
 constexpr int64_t kSplitBelow = 192;
 
 // Whether a launch at head_dim 64 or 128 takes the 128-row kernel on three-part products
-// (attention_parts.hip), by the masks and grids where it is the faster one (us, 128-row / 64-row /
-// 16-row items, 12 heads unless said):
-// - Full and Block3: 16 x 8192 Block3 78 / 112; 4 x 2048 Full 217 / 322; sequences of 768
-//   (72 items) 36.7 / 41.6 / 38.2 and 20.6 / 22.1 / 22.1, of 640 31.0 / 34.0 / 24.8.  Short
-//   sequences (few tiles an item) need more of them: 4 x 200 (96 items) 17.1 / 16.4 / 11.5, 8 x 200
-//   17.5 / 21.8 / 19.1.
-// - Sliding(w): half of an item's keys at w = 64 lie outside each wave's windows; 8 x 2048 at
-//   w = 64 73 / 70, 80 76 / 83, 128 92 / 110, 256 148 / 191, from 144 items (w = 256, 1 x 1024
-//   40.6 / 34.1 / 29.8, 1 x 1536 41.2 / 50.1 / 44.9).
+// (attention_parts.hip), by the masks and grids where it is the faster one.  Its items are twice
+// as long as the 64-row kernel's, so what it loses is a last round that few of them fill: the
+// grid is measured in rounds of one item a compute unit.  us, 128-row / 64-row / 16-row items:
+// - Full and Block3 at head_dim 64, from 144 items: 16 x 8192 Block3 78 / 112, 4 x 12 x 2048 Full
+//   208 / 322; just past a round (2 x 13 x 1161 Block3, 260 items) 31.6 / 35.1, before it
+//   (2 x 14 x 1109, 252) 22.7 / 35.3.  Fewer items are worth it on one long sequence only (12 x 768,
+//   72 items: 36.7 / 41.6 / 38.2 and 20.6 / 22.1 / 22.1; 12 x 640 31.0 / 34.0 / 24.8); in padded batches
+//   the 16-row items have less to do (3 x 8 x 388 Full 25.7 / 25.2 / 18.3).
+// - head_dim 128 (one wave a SIMD: Q's parts and the output alone fill 160 registers): Block3
+//   2 x 8 x 3000 73 / 102, Full 2 x 8 x 2048 185 / 290, from 144 items (Block3 8 x 1536, 96 items,
+//   36.3 / 35.5).  Past one round only where the rounds are 70% full: Full 23 x 3 x 442 (276 items)
+//   87 / 72, Block3 12 x 15 x 227 (360) 52 / 67.
+// - Sliding(w) from w = 128: part of an item's keys lie outside each wave's windows.  8 x 12 x 2048
+//   at w = 64 73 / 70, 128 92 / 110, 256 148 / 191; 13 x 8 x 652 at 107 48.4 / 45.6.  Past one
+//   round at 75% (8 x 5 x 1217 at 205, 400 items, 51 / 58); at head_dim 128 at 90% (18 x 4 x 541 at
+//   237, 360 items, 87 / 76; 4 x 8 x 2048 at 128, 512 items, 96 / 101).
 // - not BlockDiag: one or two tiles an item leave nothing to gain from cheaper products (64 is
 //   bound by memory).
-// - head_dim 128 (one wave a SIMD: Q's parts and the output alone fill 160 registers): Block3
-//   2 x 8 x 3000 83 / 99, 8 x 8 x 2048 167 / 228, Full 2 x 8 x 2048 185 / 290; from 144 items (Block3
-//   1 x 8 x 1536, 96 items, 36.3 / 35.5), Sliding from w = 128 (64: 70.5 / 68.1, 128: 96 / 101).
 // Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.
-constexpr int64_t kPartsFrom = 144, kPartsFromWide = 72;
-constexpr int64_t kWideSeq = 384, kPartsWindow = 80, kPartsWindow128 = 128;
+constexpr int64_t kPartsFrom = 144, kPartsFromAlone = 72, kAloneSeq = 768;
+constexpr int64_t kPartsWindow = 128, kRound = 256;
 
 bool takes_parts(const AttnLaunch &a) {
     const bool block = a.mask_kind == RAYA_MASK_FULL || a.mask_kind == RAYA_MASK_BLOCK3;
     const bool wide = a.head_dim > 64;
-    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= (wide ? kPartsWindow128 : kPartsWindow))) return false;
+    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= kPartsWindow)) return false;
     const int64_t tiles = (a.seq + kPartRows - 1) / kPartRows;
     if (5 * (int64_t)a.seq < 3 * kPartRows * tiles) return false;  // under 60% of the items' rows
-    return tiles * a.heads * a.batch >= (block && !wide && a.seq >= kWideSeq ? kPartsFromWide : kPartsFrom);
+    const int64_t items = tiles * a.heads * a.batch;
+    if (items < (block && !wide && a.batch == 1 && a.seq >= kAloneSeq ? kPartsFromAlone : kPartsFrom)) return false;
+    const int64_t percent = wide ? (block ? 70 : 90) : (block ? 0 : 75);
+    const int64_t rounds = (items + kRound - 1) / kRound;
+    return rounds == 1 || 100 * items >= percent * rounds * kRound;
 }
 
 // Query rows of an item.  RAYA_ATTN_ITEMS=16, 64 or 128 forces the height where the kernel
