@@ -4,10 +4,17 @@
 // a is [m, k] row-major, b is a Linear weight [n, k] row-major, so both
 // operands are contiguous along k.
 //
-// Arithmetic.  Every fp32 operand x is written as the sum of three bfloat16
+// Arithmetic.  Every fp32 operand, times 2^23 (exact), is written as the sum of three bfloat16
 // parts: x0 = x rounded to 8 bits, x1 = x - x0 rounded to 8 bits, x2 = x - x0 - x1.  Both
 // differences are exact in fp32 and the second has at most 7 bits, so x = x0 + x1 + x2
-// exactly, with |x1| <= 2^-8 |x| and |x2| <= 2^-17 |x|.  Of the nine part products the six
+// exactly, with |x1| <= 2^-8 |x| and |x2| <= 2^-17 |x|.  The scale lifts the last bit of the
+// smallest fp32 subnormal (2^-149) to bfloat16's smallest normal number: unscaled, the lower
+// parts of an operand below 2^-110 fell below bfloat16's smallest subnormal (the product was off
+// by 2e-6 at 2^-116 and 6e-4 at 2^-124), and the matrix instruction aligns a subnormal part as
+// if its leading bit were set, which costs the sum up to 7 bits.  The sums leave the scale by
+// 2^-46 after the K loop.  The scaling takes 1% of a large product (QKV at 21,405 rows 380 ->
+// 384 us) and gives the same bits wherever the unscaled parts were exact.  Of the nine part
+// products the six
 // a2 b0 + a0 b2 + a1 b1 + a1 b0 + a0 b1 + a0 b0 are summed, each exact in the fp32
 // accumulator of v_mfma_f32_32x32x16_bf16; a1 b2 and a2 b1 (each at most 2^-25 of |a b|,
 // typically 2^-28) and a2 b2 are left out.  The accumulator takes 6 roundings per 16 k where
@@ -22,10 +29,11 @@
 // 367 us (207) here; 768 x 768 189 -> 127 us, GeGLU 6144 x 768 1,463 -> 920 us,
 // 768 x 3072 725 -> 443 us.
 //
-// Parts of Inf and NaN (and of |x| above the largest bfloat16) are not sums of
-// anything, so an operand that is not finite leaves every output of its row or column
-// not finite; those outputs, and only those, are computed again with the fp32
-// instruction over the unsplit operands (exact_subtile).
+// Parts of Inf and NaN (and of |x| from 2^105 on, whose scaled value is above the largest
+// bfloat16) are not sums of anything, so such an operand leaves every output of its row or column
+// not finite, and so does a scaled sum past the largest float (2^82 unscaled); those outputs, and
+// only those, are computed again with the fp32 instruction over the unsplit operands
+// (exact_subtile).
 //
 // Register layouts (lane l, half h = l / 32):
 //   v_mfma_f32_32x32x16_bf16: A[i][8h .. 8h + 7] in lane i + 32 h, B[.][j] in lane j + 32 h;
@@ -360,6 +368,9 @@ __device__ __forceinline__ floatx16 exact_subtile(const float *arow, const float
     return e;
 }
 
+// The operands' scale, and the sums'.
+constexpr float kScale = 0x1p23f, kUnscale = 0x1p-46f;
+
 // 16-byte loads of whole chunks of 4 k.
 __host__ __device__ __forceinline__ bool aligned_rows(const GemmLaunch &g) {
     return ((g.lda | g.ldb | g.k) & 3) == 0 && (((uintptr_t)g.a | (uintptr_t)g.b) & 15) == 0;
@@ -385,7 +396,7 @@ __device__ __forceinline__ int b_row(const GemmLaunch &g, int n0, int row) {
 // epilogue drops them), are split into their parts in registers and written to LDS as three
 // planes.  Iteration kt multiplies slab kt out of one stage while slab kt + 1, fetched PF
 // iterations ago, is split into the other between the MFMAs, so the splitting's VALU work
-// (5.5 operations an element) runs beside the matrix cores; one barrier per slab.
+// (6.5 operations an element) runs beside the matrix cores; one barrier per slab.
 template <class T, bool GEGLU, bool NORM, bool STATS, int PAD>
 __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaunch g) {
     __shared__ __attribute__((aligned(16))) char ring[T::LDS];
@@ -460,7 +471,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
                 const int row = min(m0 + r0 + p * RPP, g.m - 1);
                 src[p] = g.a + (int64_t)row * g.lda + 4 * c;
                 cen[p] = 0.f;
-                if constexpr (NORM) cen[p] = norm_centre(norms[r0 + p * RPP]);
+                if constexpr (NORM) cen[p] = norm_centre(norms[r0 + p * RPP]) * kScale;
             } else {
                 src[p] = g.b + (int64_t)b_row<GEGLU>(g, n0, r0 + p * RPP - T::BM) * g.ldb + 4 * c;
             }
@@ -491,18 +502,13 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
                 const int left = g.k - (slab0 + kt) * BK - 4 * c;
                 x = make_float4(left > 0 ? x.x : 0.f, left > 1 ? x.y : 0.f, left > 2 ? x.z : 0.f, left > 3 ? x.w : 0.f);
             }
-            if constexpr (NORM) {
-                if (p < APASS) {
-                    const float o = cen[p < APASS ? p : 0];
-                    x.x -= o;
-                    x.y -= o;
-                    x.z -= o;
-                    x.w -= o;
-                }
-            }
+            const float o = NORM && p < APASS ? cen[p < APASS ? p : 0] : 0.f;
+            const auto scaled = [&](float v) {
+                return NORM && p < APASS ? __builtin_fmaf(v, kScale, -o) : v * kScale;
+            };
             uint32_t lo[3], hi[3];
-            split3(x.x, x.y, lo);
-            split3(x.z, x.w, hi);
+            split3(scaled(x.x), scaled(x.y), lo);
+            split3(scaled(x.z), scaled(x.w), hi);
             const int r = r0 + p * RPP;
             char *d = ring + (kt & 1) * T::STAGE + ((r >> 5) * KS + (chunk >> 1)) * 1024 + (chunk & 1) * 512 +
                       ((r & 31) ^ lds_swizzle<T>(chunk)) * 16 + (c & 1) * 8;
@@ -609,7 +615,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) y[i][j][r] = acc[i][j][r];
+            for (int r = 0; r < 16; ++r) y[i][j][r] = acc[i][j][r] * kUnscale;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll

@@ -71,6 +71,59 @@ def test_operands_over_the_whole_exponent_range(hip_gemm, m, n, k):
     check(out, a, b)
 
 
+@pytest.mark.parametrize("m,n,k", [(40, 70, 2), (40, 70, 3), (33, 65, 20), (300, 200, 96), (2100, 2300, 64)])
+@pytest.mark.parametrize("exponent", [-149, -133, -126, -118, -110, -100])
+def test_tiny_operands(hip_gemm, m, n, k, exponent):
+    """Operands from 2^exponent down, subnormals among them, times operands of about 2^80 (no
+    output is subnormal): all their bits count, on either side."""
+    gen = torch.Generator(device="cuda").manual_seed(k - exponent)
+    for swap in (False, True):
+        tiny = torch.randn(n if swap else m, k, device="cuda", dtype=torch.float64, generator=gen)
+        tiny = (tiny * 2.0 ** exponent).float()
+        big = torch.randn(m if swap else n, k, device="cuda", generator=gen) * 2.0 ** 80
+        a, b = (big, tiny) if swap else (tiny, big)
+        out = torch.empty(m, n, device="cuda")
+        hip_gemm.matmul_nt_device(out, a, b)
+        check(out, a, b)
+
+
+def test_tiny_weights_behind_a_folded_norm(hip_gemm):
+    """Weights of about 2^-122 and rows normalised on the way in: within the bound around the
+    64-bit product of the normalised rows, whose own rounding adds one unit per product."""
+    m, n, k = 70, 132, 16
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    x = 2.0 + torch.randn(m, k, device="cuda", generator=gen)
+    b = (torch.randn(n, k, device="cuda", generator=gen).double() * 2.0 ** -122).float()
+    mean, rstd = x.double().mean(1), 1.0 / x.double().std(1, unbiased=False)
+    rows = torch.zeros(m, 4, device="cuda")
+    rows[:, 0] = mean.float()
+    rows[:, 1] = (mean - mean.float().double()).float()
+    rows[:, 2] = rstd.float()
+    sums = torch.empty(n, device="cuda")
+    hip_gemm.weight_row_sums(b, sums)
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, x, b, in_row_stats=rows, in_weight_sums=sums)
+    norm = (x.double() - mean[:, None]) * rstd[:, None]
+    want = norm @ b.double().T
+    bound = (2 * k + 8) * 2.0 ** -24 * (norm.abs() @ b.double().abs().T)
+    worst = float(((out.double() - want).abs() / bound).max())
+    assert worst <= 1, worst
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 70, 3), (300, 200, 96), (2100, 2300, 64)])
+@pytest.mark.parametrize("ea,eb", [(100, -100), (104, -60), (106, -106), (120, -120), (41, 40), (70, 45)])
+def test_large_operands_and_sums(hip_gemm, m, n, k, ea, eb):
+    """Finite operands from about 2^105, whose scaled parts overflow, and finite sums from about
+    2^82, on either side of both lines."""
+    gen = torch.Generator(device="cuda").manual_seed(ea)
+    a = torch.randn(m, k, device="cuda", generator=gen) * 2.0 ** ea
+    b = torch.randn(n, k, device="cuda", generator=gen) * 2.0 ** eb
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, a, b)
+    assert torch.isfinite(out).all()
+    check(out, a, b)
+
+
 @pytest.mark.parametrize("m,n,k", [(40, 70, 96), (300, 200, 100), (2100, 2300, 64)])
 def test_non_finite_operands(hip_gemm, m, n, k):
     """Inf, NaN and 3.4e38 in single elements of a and b: NaN and Inf where the reference has
