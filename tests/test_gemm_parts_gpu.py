@@ -110,6 +110,18 @@ def test_tiny_weights_behind_a_folded_norm(hip_gemm):
     assert worst <= 1, worst
 
 
+@pytest.mark.parametrize("m,n", [(1, 1), (40, 70), (300, 200), (2100, 2300)])
+@pytest.mark.parametrize("exponent", [0, -100, 100])
+def test_depth_one_is_the_rounded_product(hip_gemm, m, n, exponent):
+    """One product has one rounding."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    a = torch.randn(m, 1, device="cuda", generator=gen) * 2.0 ** exponent
+    b = torch.randn(n, 1, device="cuda", generator=gen)
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, a, b)
+    assert torch.equal(out, a * b.reshape(1, n))
+
+
 @pytest.mark.parametrize("m,n,k", [(40, 70, 3), (300, 200, 96), (2100, 2300, 64)])
 @pytest.mark.parametrize("ea,eb", [(100, -100), (104, -60), (106, -106), (120, -120), (41, 40), (70, 45)])
 def test_large_operands_and_sums(hip_gemm, m, n, k, ea, eb):
