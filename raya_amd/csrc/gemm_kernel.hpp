@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
                 src[p] = g.b + (int64_t)b_row<GEGLU>(g, n0, r0 + p * RPP - T::BM) * g.ldb + 4 * c;
             }
         }
-        const int slabs = (g.k + BK - 1) / BK;
+        const int slabs = g.k / BK + (g.k % BK != 0);
         const int slab0 = (int)((int64_t)slabs * split / S), nk = (int)((int64_t)slabs * (split + 1) / S) - slab0;
         float4 st[PF][PASS];
         const auto load = [&](int kt, float4 (&x)[PASS]) {
@@ -499,7 +499,7 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
         };
         const auto put = [&](int kt, int p, float4 x) {
             if constexpr (PAD != 0) {
-                const int left = g.k - (slab0 + kt) * BK - 4 * c;
+                const int left = (int)((uint32_t)g.k - (uint32_t)(slab0 + kt) * BK) - 4 * c;
                 x = make_float4(left > 0 ? x.x : 0.f, left > 1 ? x.y : 0.f, left > 2 ? x.z : 0.f, left > 3 ? x.w : 0.f);
             }
             const float o = NORM && p < APASS ? cen[p < APASS ? p : 0] : 0.f;

@@ -110,6 +110,20 @@ def test_tiny_weights_behind_a_folded_norm(hip_gemm):
     assert worst <= 1, worst
 
 
+@pytest.mark.parametrize("m,n,k", [(268435456 + 77, 1, 2), (128 * (0x7FFFFFFF // 256), 1, 1), (3, 300000001, 1)])
+def test_very_tall_and_wide_outputs(hip_gemm, m, n, k):
+    """Grids past 2^22 workgroups; rows and columns checked at both ends and in between."""
+    a = torch.arange(m * k, device="cuda", dtype=torch.int32).remainder_(4093).float().reshape(m, k)
+    b = torch.arange(n * k, device="cuda", dtype=torch.int32).remainder_(61).float().reshape(n, k)
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, a, b)
+    for r0 in range(0, m, max(1, m // 7)):
+        for c0 in range(0, n, max(1, n // 7)):
+            x, y = a[r0:r0 + 2000], b[c0:c0 + 2000]
+            assert torch.equal(out[r0:r0 + 2000, c0:c0 + 2000], x @ y.T)
+    assert torch.equal(out[-300:, -300:], a[-300:] @ b[-300:].T)
+
+
 @pytest.mark.parametrize("m,n", [(1, 1), (40, 70), (300, 200), (2100, 2300)])
 @pytest.mark.parametrize("exponent", [0, -100, 100])
 def test_depth_one_is_the_rounded_product(hip_gemm, m, n, exponent):
