@@ -354,18 +354,67 @@ template <class T>
 __device__ __forceinline__ int lds_swizzle(int chunk) { return T::KS <= 4 ? chunk * (4 / T::KS) : chunk & 7; }
 
 // One 32 x 32 output subtile in fp32 from the unsplit operands, for outputs that the parts
-// left not finite: the lane's A row (less its folded-norm centre) and B row.
-__device__ __forceinline__ floatx16 exact_subtile(const float *arow, const float *brow, int k, int h, float cen) {
-    floatx16 e;
+// left not finite: the lane's A row (less its folded-norm centre) and B row, in the order of k
+// (infinities of either sign in a row meet in the reference's order).  32 k are fetched ahead of the
+// products (96: no faster, and spills).  Of rows of 16-byte chunks (VEC) a lane takes 4 consecutive k
+// of each 8, half h from 4 h on, and the halves exchange elements to make operands of consecutive k.
+// With single loads per k and two of them in flight, 21,405 x 2304 x 768 of NaN took 4,273 us, with Inf
+// in every 64th row 2,351 and with one NaN in b 714; now 1,334, 870 and 595 (all finite 378).
+template <bool VEC>
+__device__ __forceinline__ floatx16 exact_subtile(const float *arow, const float *brow, int depth, uint32_t h, float cen) {
+    constexpr uint32_t SPAN = 32;
+    const uint32_t k = depth;
+    const auto load = [&](const float *row, uint32_t t0, float (&x)[SPAN / 2]) {
+        if constexpr (VEC) {  // k is a multiple of 4
 #pragma unroll
-    for (int r = 0; r < 16; ++r) e[r] = 0.f;
-#pragma unroll 4
-    for (int t = 0; t < k; t += 2) {
-        const int kt = min(t + h, k - 1);
-        const float x = arow[kt] - cen, y = brow[kt];
-        e = mfma_f32(t + h < k ? x : 0.f, t + h < k ? y : 0.f, e);
+            for (uint32_t s = 0; s < SPAN / 8; ++s) {
+                const float4 u = *(const float4 *)(row + min(t0 + 8 * s + 4 * h, k - 4));
+                x[4 * s] = u.x, x[4 * s + 1] = u.y, x[4 * s + 2] = u.z, x[4 * s + 3] = u.w;
+            }
+        } else {
+#pragma unroll
+            for (uint32_t p = 0; p < SPAN / 2; ++p) x[p] = row[min(t0 + 2 * p + h, k - 1)];
+        }
+    };
+    // x[p]: the element of k = t0 + 2 p + h.
+    const auto order = [&](float (&x)[SPAN / 2]) {
+        if constexpr (VEC) {
+            const auto swap = [](float &lo, float &hi) {
+                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(lo), __float_as_uint(hi), false, false);
+                lo = __uint_as_float(r[0]);
+                hi = __uint_as_float(r[1]);
+            };
+#pragma unroll
+            for (uint32_t s = 0; s < SPAN / 2; s += 4) {
+                swap(x[s], x[s + 1]);
+                swap(x[s + 2], x[s + 3]);
+                const float t = x[s + 1];
+                x[s + 1] = x[s + 2];
+                x[s + 2] = t;
+            }
+        }
+    };
+    floatx16 y;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) y[r] = 0.f;
+    if (k == 0) return y;
+    float a[SPAN / 2], b[SPAN / 2], an[SPAN / 2], bn[SPAN / 2];
+    load(arow, 0, an);
+    load(brow, 0, bn);
+    for (uint32_t t0 = 0; t0 < k; t0 += SPAN) {
+#pragma unroll
+        for (uint32_t p = 0; p < SPAN / 2; ++p) a[p] = an[p], b[p] = bn[p];
+        load(arow, t0 + SPAN, an);
+        load(brow, t0 + SPAN, bn);
+        order(a);
+        order(b);
+#pragma unroll
+        for (uint32_t p = 0; p < SPAN / 2; ++p) {
+            const bool in = t0 + 2 * p + h < k;
+            y = mfma_f32(in ? a[p] - cen : 0.f, in ? b[p] : 0.f, y);
+        }
     }
-    return e;
+    return y;
 }
 
 // The operands' scale, and the sums'.
@@ -614,31 +663,37 @@ __global__ void __launch_bounds__(T::THREADS, T::OCC) gemm_kernel(const GemmLaun
     const bool exact = g.k == 1;
     // From here on single floats: a 16-register vector changed in a branch would be held twice.
     float y[TM][2][16];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) y[i][j][r] = acc[i][j][r] * kUnscale;
+    uint32_t redo = 0;  // subtiles 2 i + j with outputs to compute again
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            bool bad = exact;
+            float z = 0.f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) bad |= !(fabsf(y[i][j][r]) <= 3.40282347e38f);
-            if (__any(bad)) {
-                const int row = min(m0 + wm + 32 * i + li, g.m - 1);
-                float cen = 0.f;
-                if constexpr (NORM) cen = norm_centre(norms[wm + 32 * i + li]);
-                const floatx16 e =
-                    exact_subtile(g.a + (int64_t)row * g.lda,
-                                  g.b + (int64_t)b_row<GEGLU>(g, n0, wn + 32 * j + li) * g.ldb, g.k, h, cen);
-#pragma unroll
-                for (int r = 0; r < 16; ++r)
-                    if (exact || !(fabsf(y[i][j][r]) <= 3.40282347e38f)) y[i][j][r] = e[r];
+            for (int r = 0; r < 16; ++r) {
+                y[i][j][r] = acc[i][j][r] * kUnscale;
+                z = __builtin_fmaf(y[i][j][r], 0.f, z);  // NaN where one of them is not finite
             }
+            if (exact || __any(z != 0.f)) redo |= 1u << (2 * i + j);
         }
+    // One copy of the code for all of them: a copy each made every launch 1-2% slower.
+    while (redo) {
+        const int at = __builtin_ctz(redo), i = at >> 1, j = at & 1;
+        redo &= redo - 1;
+        const int row = min(m0 + wm + 32 * i + li, g.m - 1);
+        float cen = 0.f;
+        if constexpr (NORM) cen = norm_centre(norms[wm + 32 * i + li]);
+        const floatx16 e = exact_subtile<PAD != 2>(
+            g.a + (int64_t)row * g.lda, g.b + (int64_t)b_row<GEGLU>(g, n0, wn + 32 * j + li) * g.ldb, g.k, h, cen);
+#pragma unroll
+        for (int q = 0; q < 2 * TM; ++q)
+            if (q == at)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float &x = y[q >> 1][q & 1][r];
+                    x = exact || !(fabsf(x) <= 3.40282347e38f) ? e[r] : x;
+                }
+    }
 
     const bool vec_out = (g.ldo & 3) == 0 && ((uintptr_t)g.out & 15) == 0 &&
                          (!g.residual || ((g.ldr & 3) == 0 && ((uintptr_t)g.residual & 15) == 0));

@@ -185,3 +185,21 @@ def test_non_finite_operands(hip_gemm, m, n, k):
     keep[rows] = False
     keep[:, cols] = False
     assert np.array_equal(got[keep], plain.cpu().numpy()[keep])
+
+
+@pytest.mark.parametrize("k", [1, 2, 5, 31, 32, 33, 64, 100, 131])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_exact_outputs_at_every_depth(hip_gemm, k, offset):
+    """Rows whose parts overflow (values from 2^120) are computed from the unsplit operands: every
+    remainder of the 32 k that a step takes, of aligned rows and of rows one float past a boundary."""
+    m, n = 70, 66
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    a = torch.zeros(m, k + 4 - k % 4 + 4, device="cuda")[:, offset:k + offset]
+    b = torch.zeros(n, k + 4 - k % 4 + 4, device="cuda")[:, offset:k + offset]
+    a.copy_(torch.randn(m, k, device="cuda", generator=gen))
+    b.copy_(torch.randn(n, k, device="cuda", generator=gen) * 2.0 ** -60)
+    a[::3] *= 2.0 ** 120
+    out = torch.empty(m, n, device="cuda")
+    hip_gemm.matmul_nt_device(out, a, b)
+    assert torch.isfinite(out).all()
+    check(out, a, b)
