@@ -663,13 +663,11 @@ __device__ __forceinline__ void lap(StageClock *c, uint64_t &bucket) {
 // MK >= 0: the mask kind is fixed at compile time; SINGLE: every item's keys fit one
 // tile (BlockDiag(b) with b dividing 64).  Both only drop code the launch has ruled out.
 //
-// REDO: only outputs that are not finite now are written (attention_parts.hip's second pass).
-//
 // MAXT > 0 (the direct path, items of at most MAXT tiles): every tile's K/V subtile
 // is loaded into registers before the first is computed, so the tile loads' latencies
 // overlap each other rather than each one the previous tile's arithmetic.
 template <int DP, bool FUSED, bool TIMED, bool SKIP = false, bool SPLIT = false, int MK = -1,
-          bool SINGLE = false, int MAXT = 0, bool EXACTV = true, bool REDO = false>  // head_dim padded to a multiple of 16
+          bool SINGLE = false, int MAXT = 0, bool EXACTV = true>  // head_dim padded to a multiple of 16
 __device__ __forceinline__ void attend_body(const AttnLaunch &a, const Plan &p, const Item &it, float *__restrict__ ks,
                                             float *__restrict__ vs, StageClock *clk) {
     static_assert(!FUSED || DP == 64, "the fused issue is written for head_dim 64");
@@ -1169,10 +1167,7 @@ __device__ __forceinline__ void attend_body(const AttnLaunch &a, const Plan &p, 
         for (int t = 0; t < 4; ++t) {
             const int r = 4 * t + (lane >> 4), c = lane & 15;
             const float4 y = *(const float4 *)(st + r * 64 + 4 * (c ^ r));
-            if (qw + r >= rows) continue;
-            float *o = ob + (int64_t)(qw + r) * a.o_rs + 4 * c;
-            if (REDO && finite4(*(const float4 *)o)) continue;
-            store_stream(o, y);
+            if (qw + r < rows) store_stream(ob + (int64_t)(qw + r) * a.o_rs + 4 * c, y);
         }
         return;
     }
@@ -1193,7 +1188,6 @@ __device__ __forceinline__ void attend_body(const AttnLaunch &a, const Plan &p, 
                 if (ragged && !zero_row && !finite4(y))
                     y = exact_chunk(a.q + base(a.q_bs, a.q_hs, a.q_rs) + (int64_t)qi * a.q_rs, kb, a.k_rs, vb,
                                     a.v_rs, rr.lo, rr.hi, D, a.scale, g * DQ + 4 * c);
-                if (REDO && finite4(*(const float4 *)(orow + 4 * c))) continue;
                 *(float4 *)(orow + 4 * c) = y;
             }
         }

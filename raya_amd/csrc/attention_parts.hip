@@ -31,8 +31,9 @@
 // matrix cores, with one barrier after each phase.  Rows are fetched into registers two phases
 // ahead.
 //
-// Outputs that are not finite (an operand that is not finite, or above the largest bfloat16,
-// has no parts) are computed again by the fp32 body in the same workgroup, and only they.
+// Halves of 64 rows with an output that is not finite (an operand that is not finite, or above the
+// largest bfloat16, has no parts) are left to the fp32 body, in the same workgroup and before
+// anything of them is stored (q may be out).
 #include "attention_body.hpp"
 #include "parts.hpp"
 
@@ -375,26 +376,26 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
             bad |= !finite4(y);
             *(float4 *)(st + li * D + 4 * ((8 * t + 2 * r + h) ^ (li & 15))) = y;
         }
+    int redo = 0;  // halves
+    if (__syncthreads_or(bad)) redo = (__syncthreads_or(bad && wave < 2) ? 1 : 0) | (__syncthreads_or(bad && wave >= 2) ? 2 : 0);
     const int rows = packed ? valid : a.seq;
+    if (!(redo >> (wave >> 1) & 1)) {
 #pragma unroll
-    for (int i = 0; i < CH / 2; ++i) {
-        const int at = i * 64 + lane, r = at / CH, c = at % CH;
-        const float4 y = *(const float4 *)(st + r * D + 4 * (c ^ (r & 15)));
-        if (qw + r < rows) store_stream(ob + (int64_t)(qw + r) * a.o_rs + 4 * c, y);
-    }
-    if (__syncthreads_or(bad)) {
-        // (The barrier's fence has the stores done and the staging read.)
-        __threadfence();
-#pragma unroll 1
-        for (int q0 = it.q0; q0 < min(it.q0 + kPartRows, valid); q0 += kQRows) {
-            Item half_item = it;
-            half_item.q0 = q0;
-            half_item.k_lo = key_range(MK, arg, p.by_arg, q0, valid).lo;
-            half_item.k_hi = key_range(MK, arg, p.by_arg, min(q0 + kQRows, valid) - 1, valid).hi;
-            attend_body<D, D == 64, false, WINDOW && D == 64, false, MK, false, 0, WINDOW, true>(a, p, half_item, (float *)lds,
-                                                                                  (float *)lds + kKeys * D, nullptr);
-            __syncthreads();
+        for (int i = 0; i < CH / 2; ++i) {
+            const int at = i * 64 + lane, r = at / CH, c = at % CH;
+            const float4 y = *(const float4 *)(st + r * D + 4 * (c ^ (r & 15)));
+            if (qw + r < rows) store_stream(ob + (int64_t)(qw + r) * a.o_rs + 4 * c, y);
         }
+    }
+#pragma unroll 1
+    for (; redo; redo &= redo - 1) {
+        Item half_item = it;
+        half_item.q0 = it.q0 + (redo & 1 ? 0 : kQRows);
+        half_item.k_lo = key_range(MK, arg, p.by_arg, half_item.q0, valid).lo;
+        half_item.k_hi = key_range(MK, arg, p.by_arg, min(half_item.q0 + kQRows, valid) - 1, valid).hi;
+        __syncthreads();
+        attend_body<D, D == 64, false, WINDOW && D == 64, false, MK, false, 0, WINDOW>(
+            a, p, half_item, (float *)lds, (float *)lds + kKeys * D, nullptr);
     }
 }
 

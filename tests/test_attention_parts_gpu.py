@@ -157,3 +157,20 @@ def test_stages(hip_attention, name, d):
                     meets = any(t < z.stop and t + 32 > a.start for t in (kt, kt + 32))
                     n += (2 if w + 16 < v else 1) if meets else 0
     assert st.tiles == n * heads
+
+
+@pytest.mark.parametrize("name", ["block3", "full", "sliding200"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_out_may_be_q(hip_attention, name, d):
+    """q overwritten by its own outputs, some of them not finite: the same bits as in a separate out."""
+    h, s = 3, 300
+    q, k, v = (torch.from_numpy(x[None]).cuda() for x in inputs(11, h, s, d))
+    q[0, 0, 70, 1] = float("nan")
+    q[0, 1, 129, 0] = float("inf")
+    v[0, 2, 40, 3] = float("nan")
+    valid = torch.tensor([290], dtype=torch.int32, device="cuda")
+    out = torch.full_like(q, 7.0)
+    hip_attention.attend_batched(q, k, v, out, valid, MASKS[name][0], 0.125)
+    assert not torch.isfinite(out).all()
+    hip_attention.attend_batched(q, k, v, q, valid, MASKS[name][0], 0.125)
+    assert torch.equal(q.view(torch.int32), out.view(torch.int32))
