@@ -31,15 +31,29 @@
 // matrix cores, with one barrier after each phase.  Rows are fetched into registers two phases
 // ahead.
 //
-// Halves of 64 rows with an output that is not finite (an operand that is not finite, or above the
-// largest bfloat16, has no parts) are left to the fp32 body, in the same workgroup and before
-// anything of them is stored (q may be out).
+// What the parts lose, a half of 64 rows leaves to the fp32 body, in the same workgroup and before
+// anything of it is stored (q may be out):
+// - an output that is not finite: an operand that is not finite, or above the largest bfloat16, has no
+//   parts;
+// - operands so small that their lower parts fall below bfloat16's smallest subnormal, where a part is
+//   off by up to 2^-134 whatever its size.  In K that moves a score by up to 2^-134 |q| a dim, so
+//   |q scale| has to be below kHugeQ; in Q by 2^-134 |k|, so a Q element has to be zero or at least kTinyQ; in
+//   V and the weights it moves an output by up to 2^-134 (1 + |v|) a key, so V has to be below kHugeV
+//   and an output at least kTinyOut (2^-94 a key against 2^-40) or zero in a row that is not all zeros.
+// The checks take 2-3% (Block3 16 x 8192 70.8 -> 73.0 us, head_dim 128 2 x 8 x 3000 74.2 -> 76.1), half of it
+// V's largest element.  Scaling K, V and the weights as the GEMM does, which loses nothing, takes an
+// operation an element: 75.0 -> 80.2 us without the weights.
 #include "attention_body.hpp"
 #include "parts.hpp"
 
 namespace raya {
 namespace attn {
 namespace {
+
+// Orders the values that are not zero by size, zero above all of them.
+__device__ __forceinline__ uint32_t small_key(float x) { return 2 * __float_as_uint(x) - 1; }
+
+constexpr float kTinyQ = 0x1p-100f, kHugeQ = 0x1p90f, kHugeV = 0x1p40f, kTinyOut = 0x1p-40f;
 
 // acc[i] += a[i] b over the parts, the smallest products first; the sums alternate, so that
 // no instruction waits for the one before it.
@@ -174,6 +188,7 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
         for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * PLANE) = uint32x2{lo[q], hi[q]};
     };
     // Dim 64 (i / 4) + 4 dq + i % 4 of this thread's four keys.
+    float vmax = 0.f;
     const auto put_v = [&](int i) {
         const auto at = [&](int k) {
             const float4 &x = vreg[i / 4 * 4 + k];
@@ -182,6 +197,9 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
         uint32_t lo[3], hi[3];
         split3(at(0), at(1), lo);
         split3(at(2), at(3), hi);
+        // (fmaxf(fmaxf()) of these took head_dim 128 to 81 us.)
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(vmax) : "v"(at(0)), "v"(at(1)));
+        asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(vmax) : "v"(at(2)), "v"(at(3)));
         char *d = vl + v_slot(64 * (i / 4) + 4 * dq + i % 4, vs, vh) + half * 8;
 #pragma unroll
         for (int q = 0; q < 3; ++q) *(uint32x2 *)(d + q * PLANE) = uint32x2{lo[q], hi[q]};
@@ -192,12 +210,19 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
     // Q's parts: dims 16 s + 8 h .. + 7 of this lane's row (rows at or beyond valid take the last
     // one's, and all their keys are masked), negated for a negative scale.
     bf16x8 qf[DS][3];
+    uint32_t q_lo = ~0u;
+    float q_hi = 0.f;
     {
         const float *qp = a.q + base(a.q_bs, a.q_hs, a.q_rs) + (int64_t)min(qi, valid - 1) * a.q_rs + 8 * h;
 #pragma unroll
         for (int s = 0; s < DS; ++s) {
             const float4 x = *(const float4 *)(qp + 16 * s), y = *(const float4 *)(qp + 16 * s + 4);
             const float e[8] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int c = 0; c < 8; c += 2) {
+                q_lo = min(q_lo, min(small_key(e[c]), small_key(e[c + 1])));
+                q_hi = fmaxf(q_hi, fmaxf(fabsf(e[c]), fabsf(e[c + 1])));
+            }
             uint32x4 w[3];
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
@@ -364,7 +389,10 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
     float *st = (float *)lds + wave * 32 * D;
     const bool zero_row = qi >= valid || l == 0.f;
     const float inv = zero_row ? 0.f : 1.f / l;
-    bool bad = false;
+    const bool bad_v = vmax >= kHugeV;
+    bool bad = q_lo < small_key(kTinyQ) || !(q_hi * fmaxf(1.f, fabsf(a.scale)) < kHugeQ);
+    uint32_t out_lo = ~0u;
+    float out_nan = 0.f;
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -373,11 +401,17 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
             if (!zero_row)
                 y = make_float4(oacc[t][4 * r] * inv, oacc[t][4 * r + 1] * inv, oacc[t][4 * r + 2] * inv,
                                 oacc[t][4 * r + 3] * inv);
-            bad |= !finite4(y);
+            out_lo = min(min(out_lo, min(small_key(y.x), small_key(y.y))), min(small_key(y.z), small_key(y.w)));
+            out_nan = __builtin_fmaf(y.x, 0.f, __builtin_fmaf(y.y, 0.f, __builtin_fmaf(y.z, 0.f, __builtin_fmaf(y.w, 0.f, out_nan))));
             *(float4 *)(st + li * D + 4 * ((8 * t + 2 * r + h) ^ (li & 15))) = y;
         }
+    if (!zero_row) bad |= out_lo < small_key(kTinyOut) || out_lo == ~0u || out_nan != 0.f;
     int redo = 0;  // halves
-    if (__syncthreads_or(bad)) redo = (__syncthreads_or(bad && wave < 2) ? 1 : 0) | (__syncthreads_or(bad && wave >= 2) ? 2 : 0);
+    if (__syncthreads_or(bad || bad_v)) {
+        redo = (__syncthreads_or(bad && wave < 2) ? 1 : 0) | (__syncthreads_or(bad && wave >= 2) ? 2 : 0);
+        if (__syncthreads_or(bad_v)) redo = 3;
+        if (it.q0 + kQRows >= valid) redo &= 1;  // the second half has padding only, stored as zeros
+    }
     const int rows = packed ? valid : a.seq;
     if (!(redo >> (wave >> 1) & 1)) {
 #pragma unroll

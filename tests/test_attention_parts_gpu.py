@@ -174,3 +174,45 @@ def test_out_may_be_q(hip_attention, name, d):
     assert not torch.isfinite(out).all()
     hip_attention.attend_batched(q, k, v, q, valid, MASKS[name][0], 0.125)
     assert torch.equal(q.view(torch.int32), out.view(torch.int32))
+
+
+@pytest.mark.parametrize("name", list(MASKS))
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("eq,ek,ev", [(0, 0, -120), (124, -124, 0), (-124, 124, 0), (-79, 79, 0), (-82, 82, 0), (100, -100, 100),
+                                      (0, 0, 81), (0, 0, 120), (60, -60, -90)])
+def test_operands_of_any_size(hip_attention, name, d, eq, ek, ev):
+    """Operands of 2^eq, 2^ek and 2^ev, scores of order one: rel-L2 1e-5 around float64 as at every
+    other size (the smallest lose no bits, the largest are left to the fp32 body)."""
+    h, s, valid = 2, 300, 290
+    x = [torch.from_numpy(t[None]).cuda() * 2.0 ** e for t, e in zip(inputs(21, h, s, d), (eq, ek, ev))]
+    out = torch.full_like(x[0], 7.0)
+    hip_attention.attend_batched(*x, out, torch.tensor([valid], dtype=torch.int32, device="cuda"), MASKS[name][0], 0.125)
+    assert (out[:, :, valid:] == 0).all()
+    q, k, v = (t[0, :, :valid].double() for t in x)
+    kind, block, window = MASKS[name][1:]
+    i = torch.arange(valid, device="cuda")
+    seen = {oracle.MASK_BLOCK3: (i[:, None] // 128 - i[None] // 128).abs() <= 1, oracle.MASK_FULL: i[:, None] >= i[None] * 0,
+            oracle.MASK_SLIDING: (i[:, None] - i[None]).abs() <= window}[kind]
+    w = torch.softmax((torch.matmul(q, k.transpose(1, 2).contiguous()) * 0.125).masked_fill(~seen, -np.inf), -1)
+    want = torch.matmul(w, v) * 2.0 ** -ev
+    got = out[0, :, :valid].double() * 2.0 ** -ev
+    assert float((got - want).norm() / want.norm()) <= 1e-5
+    assert float((got - want).abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_tiny_weights_of_huge_values(hip_attention, d):
+    """Keys that weigh about 2^-112 with V of 2^104: their part of the sum counts as much as the rest."""
+    h, s = 1, 256
+    q, k, v = (torch.from_numpy(t[None]).cuda() for t in inputs(22, h, s, d))
+    q[:], k[:] = 0.0, 0.0
+    q[..., 0] = 1.0
+    k[..., ::2, 0] = -112 * float(np.log(2)) * 8 + 0.1 * k[..., ::2, 1]
+    v[..., ::2, :] *= 2.0 ** 104
+    v[..., 1::2, :] *= 2.0 ** -8
+    out = torch.full_like(q, 7.0)
+    hip_attention.attend_batched(q, k, v, out, torch.tensor([s], dtype=torch.int32, device="cuda"), R.Mask.FULL, 0.125)
+    w = torch.softmax(torch.matmul(q[0].double(), k[0].double().transpose(1, 2).contiguous()) * 0.125, -1)
+    want = torch.matmul(w, v[0].double())
+    # The exponents' own rounding: -112 with 24 bits is off by 2^-18, its weight by 2.6e-6.
+    assert float((out[0].double() - want).norm() / want.norm()) <= 2e-5
