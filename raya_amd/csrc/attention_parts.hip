@@ -108,6 +108,17 @@ __device__ __forceinline__ Item decode_longest_first(const AttnLaunch &a, const 
     return decode<kPartRows, RAYA_MASK_FULL>(a, p, item + (seq - slot) * a.heads * p.n_qt);
 }
 
+// Whole (sequence, head) pairs per XCD (item_of): the tiles of a pair start one further on than those
+// of the XCD's pair before.  An XCD deals its workgroups to four shader engines in turn, so that
+// with a multiple of four tiles a pair (two, by halves) the same engines would get every pair's padding:
+// 64 x 12 x 512 with 128 to 256 valid rows took 114 us under Full instead of 76, with 128 to 512 under
+// Block3 163 instead of 129, at head_dim 128 304 instead of 190 and 401 instead of 320.
+__device__ __forceinline__ int rotate_tiles(const Plan &p, int item) {
+    if (p.pairs_per_xcd == 0 || p.rot_units > 0) return item;
+    const int bh = fdiv(item, p.by_qt), t = item - bh * p.n_qt + bh / kXcds;
+    return bh * p.n_qt + t - fdiv(t, p.by_qt) * p.n_qt;
+}
+
 template <int D, int MK, bool TIMED>
 __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, char *lds, StageClock *clk) {
     constexpr int DS = D / 16, DT = D / 32, CH = D / 4;  // MFMA steps, 32-wide tiles and 16-byte chunks of a row
@@ -117,7 +128,7 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
     constexpr bool WINDOW = MK == RAYA_MASK_SLIDING;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int li = lane & 31, h = lane >> 5;
-    const int item = item_of(blockIdx.x, p);
+    const int item = rotate_tiles(p, item_of(blockIdx.x, p));
     const bool sorted = MK == RAYA_MASK_FULL && a.valid_len && a.batch > 1 && a.batch <= kMaxSorted;
     const Item it = sorted ? decode_longest_first(a, p, item) : decode<kPartRows, MK>(a, p, item);
     const bool packed = a.seq_start != nullptr;

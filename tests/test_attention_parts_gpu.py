@@ -216,3 +216,54 @@ def test_tiny_weights_of_huge_values(hip_attention, d):
     want = torch.matmul(w, v[0].double())
     # The exponents' own rounding: -112 with 24 bits is off by 2^-18, its weight by 2.6e-6.
     assert float((out[0].double() - want).norm() / want.norm()) <= 2e-5
+
+
+def attend(hip_attention, x, lens, mask):
+    out = torch.full_like(x[0], 7.0)
+    hip_attention.attend_batched(*x, out, torch.tensor(lens, dtype=torch.int32, device="cuda"), mask)
+    return out
+
+
+@pytest.mark.parametrize("seq", [4096, 2000, 500, 260, 100])
+@pytest.mark.parametrize("name", ["block3", "full", "sliding200"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_item_orders(hip_attention, monkeypatch, name, seq, d):
+    """Every order of the items computes each of them once: whole pairs per XCD, their tiles rotated
+    from pair to pair (32, 16, 4, 3 and 1 tiles a pair), units of 1, 2 and 4 tiles, and 7 pairs (the scattered
+    order).  The same bits as the sequences' own launches."""
+    for b, h in ((4, 2), (24, 1), (7, 1)):
+        if b * seq > 20000:
+            continue
+        lens = [seq, max(1, seq // 3), 0, min(seq, 129), min(seq, 128), 1, seq - 1][:b] + [seq // 2] * (b - 7)
+        x = [torch.from_numpy(synth.normal(31 + i, b * h * seq * d).reshape(b, h, seq, d)).cuda() for i in range(3)]
+        monkeypatch.delenv("RAYA_ATTN_ORDER", raising=False)
+        want = torch.cat([attend(hip_attention, [t[i:i + 1].contiguous() for t in x], lens[i:i + 1], MASKS[name][0])
+                          for i in range(b)])
+        for order in (None, "pairs", "rot1", "rot2", "rot4"):
+            if order:
+                monkeypatch.setenv("RAYA_ATTN_ORDER", order)
+            assert torch.equal(attend(hip_attention, x, lens, MASKS[name][0]), want), (b, h, order)
+
+
+@pytest.mark.parametrize("b", [2, 3, 16, 17])
+@pytest.mark.parametrize("d", [64, 128])
+def test_longest_first_at_its_limit_and_packed(hip_attention, b, d):
+    """Full batches of up to 16 sequences run longest first, ties and empty ones included; 17 do not.
+    Also read out of rows of [heads dim + 8] floats."""
+    h, s = 3, 300
+    lens = [(37 * i + 150) % 301 if i % 5 else 200 for i in range(b)]
+    lens[-1] = 0
+    x = [torch.from_numpy(synth.normal(91 + i, b * h * s * d).reshape(b, h, s, d)).cuda() for i in range(3)]
+    want = torch.cat([attend(hip_attention, [t[i:i + 1].contiguous() for t in x], lens[i:i + 1], R.Mask.FULL)
+                      for i in range(b)])
+    assert torch.equal(attend(hip_attention, x, lens, R.Mask.FULL), want)
+    width = h * d + 8
+    rows = [torch.zeros(b, s, width, device="cuda") for _ in x]
+    for r, t in zip(rows, x):
+        r[:, :, :h * d] = t.permute(0, 2, 1, 3).reshape(b, s, h * d)
+    out = torch.full((b, s, width), 9.0, device="cuda")
+    lay = (s * width, d, width)
+    hip_attention.attend_batched(*rows, out, torch.tensor(lens, dtype=torch.int32, device="cuda"), R.Mask.FULL,
+                                 layouts={"shape": (b, h, s, d), "q": lay, "k": lay, "v": lay, "out": lay})
+    assert torch.equal(out[:, :, :h * d].reshape(b, s, h, d).permute(0, 2, 1, 3), want)
+    assert (out[:, :, h * d:] == 9.0).all()
