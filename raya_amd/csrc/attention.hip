@@ -114,18 +114,23 @@ constexpr int64_t kSplitBelow = 192;
 //   87 / 72, Block3 12 x 15 x 227 (360) 52 / 67.
 // - Sliding(w) from w = 128: part of an item's keys lie outside each wave's windows.  8 x 12 x 2048
 //   at w = 64 73 / 70, 128 92 / 110, 256 148 / 191; 13 x 8 x 652 at 107 48.4 / 45.6.  Past one
-//   round at 75% (8 x 5 x 1217 at 205, 400 items, 51 / 58); at head_dim 128 at 90% (18 x 4 x 541 at
-//   237, 360 items, 87 / 76; 4 x 8 x 2048 at 128, 512 items, 96 / 101).
+//   round at 75% (8 x 5 x 1217 at 205, 400 items, 51 / 58).  At head_dim 128 from w = 256, past one round
+//   at 90% (18 x 4 x 541 at 237, 360 items, 87 / 76): 16 x 8 x 1024 of 256 to 1024 valid rows 213 / 228 at
+//   256, but 153 / 142 at 128, and 32 x 12 x 1024 at 128 402 / 383.
 // - not BlockDiag: one or two tiles an item leave nothing to gain from cheaper products (64 is
 //   bound by memory).
-// Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.
+// Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.  The lengths of a
+// device batch are not known here: with valid rows from a quarter to half of seq the 128-row kernel is
+// the faster one too (64 x 12 x 512 of 128 to 256 rows: Full 76 / 109, Block3 78 / 107, Sliding(128)
+// 76 / 99), below an eighth of seq it is not (64 x 12 x 512 of 16 to 32 rows: Full 49 / 37, Sliding(128) 43 / 28).
 constexpr int64_t kPartsFrom = 144, kPartsFromAlone = 72, kAloneSeq = 768;
-constexpr int64_t kPartsWindow = 128, kRound = 256;
+constexpr int64_t kPartsWindow = 128, kPartsWindowWide = 256, kRound = 256;
 
 bool takes_parts(const AttnLaunch &a) {
     const bool block = a.mask_kind == RAYA_MASK_FULL || a.mask_kind == RAYA_MASK_BLOCK3;
     const bool wide = a.head_dim > 64;
-    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= kPartsWindow)) return false;
+    if (!block && !(a.mask_kind == RAYA_MASK_SLIDING && a.mask_arg >= (wide ? kPartsWindowWide : kPartsWindow)))
+        return false;
     const int64_t tiles = (a.seq + kPartRows - 1) / kPartRows;
     if (5 * (int64_t)a.seq < 3 * kPartRows * tiles) return false;  // under 60% of the items' rows
     const int64_t items = tiles * a.heads * a.batch;

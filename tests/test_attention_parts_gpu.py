@@ -267,3 +267,42 @@ def test_longest_first_at_its_limit_and_packed(hip_attention, b, d):
                                  layouts={"shape": (b, h, s, d), "q": lay, "k": lay, "v": lay, "out": lay})
     assert torch.equal(out[:, :, :h * d].reshape(b, s, h, d).permute(0, 2, 1, 3), want)
     assert (out[:, :, h * d:] == 9.0).all()
+
+
+# Batch, heads, seq, head_dim, mask and the item height that a launch takes, on either side of each line.
+CHOICES = [(2, 9, 1024, 64, R.Mask.BLOCK3, "128"), (1, 143, 100, 64, R.Mask.BLOCK3, "64"), (2, 72, 100, 64, R.Mask.FULL, "128"),
+           (1, 12, 768, 64, R.Mask.FULL, "128"), (1, 12, 760, 64, R.Mask.FULL, "16"), (2, 6, 768, 64, R.Mask.FULL, "16"),
+           (1, 12, 768, 128, R.Mask.BLOCK3, "16"), (1, 18, 1024, 128, R.Mask.BLOCK3, "128"),
+           (23, 3, 442, 128, R.Mask.FULL, "64"), (23, 4, 442, 128, R.Mask.FULL, "128"),
+           (64, 3, 130, 64, R.Mask.BLOCK3, "64"), (64, 3, 200, 64, R.Mask.BLOCK3, "128"),
+           (4, 8, 1024, 64, R.Mask.sliding(128), "128"), (4, 8, 1024, 64, R.Mask.sliding(127), "64"),
+           (5, 8, 1024, 64, R.Mask.sliding(128), "64"), (6, 8, 1024, 64, R.Mask.sliding(128), "128"),
+           (4, 8, 1024, 128, R.Mask.sliding(256), "128"), (4, 8, 1024, 128, R.Mask.sliding(255), "64"),
+           (6, 8, 1024, 128, R.Mask.sliding(256), "64"), (8, 8, 1024, 128, R.Mask.sliding(256), "128"),
+           (16, 17, 300, 64, R.Mask.FULL, "128"), (17, 17, 300, 64, R.Mask.FULL, "128"),
+           (8, 12, 1024, 64, R.Mask.block_diag(128), "64"), (8, 12, 1024, 64, R.Mask.WINDOW64, "64"),
+           (8, 12, 1024, 96, R.Mask.FULL, "64")]
+
+
+@pytest.mark.parametrize("b,h,s,d,mask,rows", CHOICES)
+def test_default_dispatch(hip_attention, monkeypatch, b, h, s, d, mask, rows):
+    """What a launch takes by itself: the bits of that height forced, which on other kernels differ,
+    within the bar of the oracle on two sequences."""
+    lens = [(97 * i) % (s // 2) + s // 2 + 1 if i else s for i in range(b)]
+    x = [torch.from_numpy(synth.normal(51 + i, b * h * s * d).reshape(b, h, s, d)).cuda() for i in range(3)]
+    monkeypatch.delenv("RAYA_ATTN_ITEMS")
+    got = attend(hip_attention, x, lens, mask)
+    for forced in ("16", "64", "128"):
+        monkeypatch.setenv("RAYA_ATTN_ITEMS", forced)
+        same = torch.equal(attend(hip_attention, x, lens, mask), got)
+        no_kernel = forced == "128" and (d not in (64, 128) or mask.kind in (R.Mask.WINDOW64.kind, R.Mask.block_diag(1).kind))
+        assert same == (forced == rows) or no_kernel, (forced, same)
+    kind, block, window = {R.Mask.BLOCK3.kind: (oracle.MASK_BLOCK3, 128, 0), R.Mask.FULL.kind: (oracle.MASK_FULL, 0, 0),
+                           R.Mask.sliding(1).kind: (oracle.MASK_SLIDING, 0, mask.arg),
+                           R.Mask.WINDOW64.kind: (oracle.MASK_WINDOW64, 128, 0),
+                           R.Mask.block_diag(1).kind: (oracle.MASK_BLOCKDIAG, mask.arg, 0)}[mask.kind]
+    for i in (0, b - 1):
+        q, k, v = (t[i].cpu().numpy() for t in x)
+        want = oracle.naive_attend(q, k, v, kind, lens[i], R.kernels.default_scale(d), block=block, window=window)
+        close(got[i, :, :lens[i]].cpu().numpy(), want[:, :lens[i]])
+        assert (got[i, :, lens[i]:] == 0).all()
