@@ -89,7 +89,7 @@ hipError_t launch(const GemmLaunch &g, hipStream_t stream) {
         if (norm && (!g.colsum || (!g.in_stats && g.k % 64 != 0))) return hipErrorInvalidValue;
         if (g.out_stats && (act != kNone || g.n % 64 != 0)) return hipErrorInvalidValue;
     }
-    if (g.rope_cos && (act != kNone || g.rope_cols % kRopeHeadDim != 0 || g.rope_cols > g.n))
+    if (g.rope_cos && (act != kNone || g.residual || g.rope_cols % kRopeHeadDim != 0 || g.rope_cols > g.n))
         return hipErrorInvalidValue;
     if (g.reduce || g.splits > 1) return hipErrorInvalidValue;  // launch_gemm's own fields
     if (!within_limits(g.m, g.n, act)) return hipErrorInvalidValue;

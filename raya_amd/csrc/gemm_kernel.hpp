@@ -217,7 +217,7 @@ __device__ __forceinline__ void epilogue_staged(const GemmLaunch &g, const float
             // multiple of 64), so a lane takes the 16-byte chunks c4 and c4 + 8 of a row,
             // columns c .. c + 3 and c + 32 .. c + 35 with c = 4 c4, and rotates each pair
             // at frequencies c .. c + 3: one float4 of each table per 8 outputs.  Bias and
-            // activation came first, the residual comes after, as in epilogue().
+            // activation came first, as in epilogue(); launch_gemm takes no residual with RoPE.
             const bool rot = c0 < g.rope_cols;  // the q and k sections: whole heads
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
@@ -243,21 +243,13 @@ __device__ __forceinline__ void epilogue_staged(const GemmLaunch &g, const float
                 for (int half = 0; half < 2; ++half) {
                     const int col = c0 + 32 * half + 4 * c4;
                     if (col >= g.n) continue;
-                    float4 v = half ? x1 : x0;
+                    const float4 v = half ? x1 : x0;
                     float *o = g.out + (int64_t)row * g.ldo + col;
-                    const float *res = g.residual ? g.residual + (int64_t)row * g.ldr + col : nullptr;
                     if (col + 4 <= g.n) {
-                        if (res) {
-                            const float4 x = *(const float4 *)res;
-                            v.x += x.x;
-                            v.y += x.y;
-                            v.z += x.z;
-                            v.w += x.w;
-                        }
                         *(float4 *)o = v;
                     } else {
                         const float e[4] = {v.x, v.y, v.z, v.w};
-                        for (int q = 0; q < 4 && col + q < g.n; ++q) o[q] = res ? e[q] + res[q] : e[q];
+                        for (int q = 0; q < 4 && col + q < g.n; ++q) o[q] = e[q];
                     }
                 }
             }

@@ -54,7 +54,7 @@ struct GemmLaunch {
     // Rotary embedding fused into a plain (RAYA_EPI_NONE) epilogue: columns below
     // rope_cols (the q and k sections of a packed QKV projection, head_dim 64)
     // are rotated in pairs (c, c + 32) at position positions[row], with
-    // cos/sin tables [position][32].  rope_cos == nullptr disables it.
+    // cos/sin tables [position][32].  No residual then.  rope_cos == nullptr disables it.
     const float *rope_cos, *rope_sin;
     const int32_t *positions;
     int32_t rope_cols;
