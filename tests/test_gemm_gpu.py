@@ -50,7 +50,7 @@ def test_nan_and_inf_propagate(hip_gemm):
 
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (3, 5, 7), (17, 9, 33), (64, 64, 64), (130, 31, 257),
                                    (256, 2304, 768), (300, 768, 3072), (129, 6144, 768),
-                                   # k = 16, 32, 48: one, two and three 16-deep slabs in the LDS ring
+                                   # k = 16, 32, 48: one, two and three steps of the matrix instruction
                                    (70, 40, 16), (70, 40, 32), (200, 130, 48)])
 def test_within_the_reordering_bound(hip_gemm, m, n, k):
     rng = np.random.default_rng(m * 7 + n)
@@ -87,8 +87,8 @@ def _dev(x):
 @pytest.mark.parametrize("residual", [False, True])
 @pytest.mark.parametrize("k", [136, 128])
 def test_device_epilogues(hip_gemm, act, residual, k):
-    """bias + activation (+ residual) against the oracle's matmul_nt and scalar ops, on both
-    kernels (k = 128: the LDS-ring kernel; k = 136: the general one)."""
+    """bias + activation (+ residual) against the oracle's matmul_nt and scalar ops, with a depth of
+    whole slabs (k = 128) and a padded one (k = 136)."""
     rng = np.random.default_rng(5)
     m, n = 200, 96
     rows_b = 2 * n if act == "geglu" else n
@@ -153,7 +153,7 @@ def test_strided_out_vector_and_scalar_epilogues_agree(hip_gemm, act, residual):
 
 def test_random_sweep_of_shapes_and_epilogues(hip_gemm):
     """40 random device GEMMs against the oracle's Reference::matmul_nt: m, n, k from 1 to
-    several hundred (k a multiple of 16 in half of them, the LDS-ring kernel), every
+    several hundred (k a multiple of 16 in half of them: fewer padded slabs), every
     activation, optional bias and residual, and row strides larger than n in a third of them.
     The bound is the reordering bound above, carried through the epilogue (GELU's slope is
     at most 1.13; GeGLU's product takes each factor's error times the other factor)."""

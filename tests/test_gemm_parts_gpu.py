@@ -5,7 +5,7 @@ whose parts do not sum to them (Inf, NaN, values above the largest bfloat16).
 Bar: the reordering bound 2 k 2^-24 sum |a b| around the float64 product
 (specs/009-gemm-backend-comparison/spec.md:24), which the sequential fp32 result meets.  The six
 part products leave out at most 2^-24 of a product and are summed smallest first, with 6
-roundings per 16 k, so they meet it for every k >= 1.  Non-finite results are compared with
+roundings per 16 k, so they meet it from k = 2 on; at k = 1 the one product is rounded once.  Non-finite results are compared with
 Reference::matmul_nt's.
 """
 import numpy as np
@@ -14,6 +14,7 @@ import torch
 
 import oracle
 from raya_amd import _capi as C
+from tests.test_gemm_plan import plan
 
 pytestmark = pytest.mark.gpu
 
@@ -29,8 +30,8 @@ def check(out, a, b):
     assert worst <= 0, worst
 
 
-# Shapes by the tile they take: 32 x 64, 64 x 64, 64 x 128, 128 x 128, 256 x 128, 256 x 256, each one
-# row and column short of a whole tile or past it, with whole and padded depths.
+# Sizes one row and column short of a whole tile or past it, with whole and padded depths (the tile and
+# depth of each are pinned further down).
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (33, 65, 128), (31, 63, 200), (257, 65, 15), (257, 2303, 768),
                                    (321, 2177, 744), (513, 2305, 768), (511, 2303, 780), (1023, 2305, 768),
                                    (1025, 2049, 100), (2047, 2305, 768), (2100, 2300, 720), (4097, 3073, 768),
@@ -43,6 +44,53 @@ def test_tile_edges(hip_gemm, m, n, k):
     hip_gemm.matmul_nt_device(out[:, :n], a, b)
     check(out[:, :n], a, b)
     assert (out[:, n:] == 9.0).all()
+
+
+NONE = C.RAYA_EPI_NONE
+# By tile (rows x weight rows), whole depths, padded ones in 16-byte chunks, and others: sizes that take it,
+# one row and one column short of a whole tile or past it.
+TILE_EDGES = [
+    (32, 64, NONE, [(31, 63, 256), (33, 65, 256), (1, 1, 256), (31, 65, 780), (33, 63, 780), (31, 63, 333), (33, 65, 333)]),
+    (64, 64, NONE, [(63, 65, 128), (65, 63, 128), (63, 65, 100), (65, 63, 132), (63, 63, 67), (65, 65, 131)]),
+    (64, 128, NONE, [(8193, 127, 128), (255, 4097, 128), (8193, 127, 100), (255, 4097, 100), (4097, 255, 67), (255, 4097, 67)]),
+    (128, 128, NONE, [(8193, 257, 256), (511, 4097, 768), (8193, 255, 780), (511, 4097, 780), (4097, 513, 333), (8193, 257, 333)]),
+    (256, 128, NONE, [(8193, 511, 256), (1023, 4097, 256), (8193, 513, 132), (1023, 4097, 780), (8193, 513, 131), (8193, 511, 333)]),
+    (256, 256, NONE, [(16383, 1023, 64), (4095, 3073, 256), (16385, 513, 768)]),
+    (32, 64, GEGLU, [(31, 33, 256), (33, 31, 256), (31, 33, 780), (33, 31, 333)]),
+    (64, 64, GEGLU, [(63, 33, 128), (65, 31, 128), (63, 33, 100), (65, 33, 67)]),
+    (64, 128, GEGLU, [(8193, 63, 128), (127, 4097, 128), (8193, 63, 100), (65, 4097, 131)]),
+    (128, 128, GEGLU, [(8193, 129, 256), (2047, 1023, 256), (8193, 127, 780), (8193, 129, 333)]),
+    (256, 128, GEGLU, [(8193, 255, 256), (511, 4097, 256), (8193, 257, 132), (8193, 257, 131)]),
+    (256, 256, GEGLU, [(16383, 511, 64), (2047, 3073, 256)]),
+]
+
+
+@pytest.mark.parametrize("rows,cols,act,m,n,k", [(r, c, a, *x) for r, c, a, sizes in TILE_EDGES for x in sizes])
+def test_every_tile_at_its_edges(hip_gemm, rows, cols, act, m, n, k):
+    """Each tile with every kind of depth it takes, plain and with a bias and a residual: the bound, carried
+    through GeGLU as in test_gemm_gpu.py (GELU's slope is at most 1.13)."""
+    assert plan(m, n, k, act, vec=k % 4 == 0)[:2] == (rows, cols)
+    gen = torch.Generator(device="cuda").manual_seed(m + n + k)
+    rows_b = 2 * n if act == GEGLU else n
+    a = torch.randn(m, k, device="cuda", generator=gen)
+    b = 0.1 * torch.randn(rows_b, k, device="cuda", generator=gen)
+    bias, res = torch.randn(rows_b, device="cuda", generator=gen), torch.randn(m, n, device="cuda", generator=gen)
+    y = a.double() @ b.double().T
+    err = 2 * k * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T)
+    for extra in (False, True):
+        out = res.clone() if extra else torch.full((m, n), 9.0, device="cuda")
+        hip_gemm.matmul_nt_device(out, a, b, bias=bias if extra else None, activation=act, residual=out if extra else None)
+        want, tol = (y + bias.double(), err + 2.0 ** -24 * (y.abs() + bias.abs())) if extra else (y, err)
+        if act == GEGLU:
+            x, g = want[:, :n], want[:, n:]
+            gx = torch.nn.functional.gelu(x)
+            tol = 1.13 * tol[:, :n] * g.abs() + (gx.abs() + 1.13 * tol[:, :n]) * tol[:, n:] + 1e-6 * (gx * g).abs()
+            want = gx * g
+        if extra:
+            want = want + res.double()
+            tol = tol + 2.0 ** -23 * (want.abs() + res.abs())
+        worst = float(((out.double() - want).abs() - tol).max())
+        assert worst <= 0, (extra, worst)
 
 
 @pytest.mark.parametrize("m,n,k", [(40, 70, 131), (600, 500, 67), (5000, 777, 333)])

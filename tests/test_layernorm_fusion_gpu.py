@@ -94,7 +94,7 @@ def test_layernorm_across_gemms_matches_the_oracle(hip_gemm, offset):
 
 
 def test_row_statistics_argument_checks(hip_gemm):
-    """Shapes the ring kernel cannot take are refused before any launch."""
+    """Depths and widths that row statistics cannot take are refused before any launch."""
     from raya_amd import UnsupportedError
 
     a = torch.zeros((8, 24), device="cuda:0")

@@ -142,7 +142,7 @@ def test_batch_matches_oracle_per_sequence(tmp_path, hidden, heads, inter):
     """hidden 256: the row-in-registers LayerNorm (rows of a multiple of 256 floats); hidden 96:
     not a multiple of 64, so the LayerNorms stay kernels of their own (the others fold them
     into the GEMMs); intermediate size 200: not a multiple of 16, so the MLP's output GEMM
-    (depth 200) leaves the ring kernel and the norms stay unfolded."""
+    pads its depth and the norms stay unfolded."""
     cfg, cdir, w = make_model(tmp_path, hidden, heads, inter=inter)
     model = M.Model.load(cdir)
     rng = np.random.default_rng(hidden)
@@ -261,6 +261,31 @@ def test_base_width_layers_match_oracle(tmp_path):
             assert err.max() <= 1e-4 and rel <= 1e-5, (i, name, float(err.max()), rel)
         assert np.abs(out.logits[i] - want.logits).max() <= LAYER_TOL
         assert np.abs(out.probabilities[i] - want.probabilities).max() <= 5e-6
+
+
+def test_split_k_in_every_epilogue(tmp_path):
+    """16 tokens at hidden 1,024 and intermediate size 256: the QKV GEMM (folded norm, RoPE), the GeGLU
+    GEMM (folded norm) and the Wo GEMM (residual, row statistics) divide their depth among workgroups and
+    sum the partials in a second launch, the MLP's output GEMM at 3,072.  Bars as at the base width."""
+    from tests.test_gemm_plan import plan
+
+    d, room = 1024, 1 << 40
+    for inter, heads in ((256, 16), (3072, 16)):
+        n_splits = {"qkv": plan(16, 3 * d, d, 0, True, True, room)[3], "wo": plan(16, d, d, 0, True, True, room)[3],
+                    "geglu": plan(16, inter, d, 3, True, True, room)[3], "mlp_wo": plan(16, d, inter, 0, True, True, room)[3]}
+        assert all(n_splits[x] > 1 for x in (("qkv", "wo", "geglu") if inter == 256 else ("qkv", "wo", "mlp_wo"))), n_splits
+        cfg, cdir, w = make_model(tmp_path, d, heads, layers=2, inter=inter, head_layers=0, vocab=100, seed=31)
+        model = M.Model.load(cdir)
+        rng = np.random.default_rng(32)
+        ids, valid, pos, mask, qtype = random_batch(rng, cfg, b=1, seq=16, k=2)
+        out = model.forward_batch(ids, valid, pos, mask, qtype)
+        want = F.forward(cfg, w, ids[0], 16, pos[0], mask[0], int(qtype[0]))
+        for name in ("logits", "probabilities", "act_logits", "features", "pooled"):
+            got, exp = getattr(out, name)[0].astype(np.float64), np.asarray(getattr(want, name), np.float64)
+            err = np.abs(got - exp)
+            rel = float(np.sqrt((err ** 2).sum() / max((exp ** 2).sum(), 1e-30)))
+            print(f"  inter {inter} {name}: max-abs {err.max():.2e} rel-L2 {rel:.2e}")
+            assert err.max() <= 1e-4 and rel <= 1e-5, (inter, name, float(err.max()), rel)
 
 
 @pytest.mark.parametrize("case", ["medium", "padded"])

@@ -156,10 +156,10 @@ def test_twelve_layer_encoder_batch_order_and_size(tmp_path):
 
 @pytest.mark.timeout(600)
 def test_split_k_forward_matches_the_unsplit_batch(tmp_path):
-    """One sequence alone (few rows: every encoder GEMM and the act head split K into partial
-    tiles and a reducing launch) against the same sequence inside the bench's batch of 64
-    (thousands of rows: no GEMM splits), every output at the fp32 bar; and the split forward
-    run twice gives the same bits (the partials are summed in a fixed order)."""
+    """One sequence alone (few rows: the MLP's output GEMM splits K into partial tiles and a
+    reducing launch; test_model_gpu.py splits the others) against the same sequence inside the
+    bench's batch of 64 (thousands of rows: no GEMM splits), every output at the fp32 bar; and
+    the split forward run twice gives the same bits (the partials are summed in a fixed order)."""
     spec = W.ENCODER
     ckpt = str(tmp_path / "enc")
     checkpoint.write_synthetic(ckpt, seed=W.ENCODER_WEIGHT_SEED)
