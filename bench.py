@@ -73,9 +73,8 @@ from raya_amd.workloads import (ATTENTION as WORKLOADS, DEFAULT_ATTENTION as DEF
 PEAK_HBM_GBS = 8000.0
 PEAK_FP32_MFMA_TFLOPS = 157.3
 # An fp32 product taken as six bfloat16 part products (dense bfloat16 peak 2.5 PFLOP/s): the GEMMs
-# and the attention launches of THREE_PART; the others run on the fp32 matrix instruction.
+# and the attention launches that take 128-row items; the others run on the fp32 matrix instruction.
 PEAK_PARTS_MFMA_TFLOPS = 2500.0 / 6
-THREE_PART = {n for n, w in WORKLOADS.items() if w["mask"][0] == "block3" and w["batch"] * w["heads"] * w["seq"] >= 2 ** 15}
 METRIC = "fp32 block-local attn TFLOP/s + % roofline; encoder sequences/sec, 1 GPU"
 RAMP_MS = 60.0
 GRAPH_LAUNCHES = 20
@@ -230,8 +229,14 @@ def traffic_for(workload: str) -> dict | None:
 
 
 def mfma_peak(workload: str) -> float:
-    """TFLOP/s of fp32 products on the matrix instruction the workload's kernel uses."""
-    return PEAK_PARTS_MFMA_TFLOPS if workload in THREE_PART else PEAK_FP32_MFMA_TFLOPS
+    """TFLOP/s of fp32 products on the matrix instruction of the kernel that the library chooses."""
+    from raya_amd import _capi
+
+    w = WORKLOADS[workload]
+    mask = kernel_mask(w["mask"])
+    rows = _capi.lib().raya_attention_item_rows(w["batch"], w["heads"], w["seq"], w["head_dim"], mask.kind,
+                                                min(mask.arg, w["seq"]))
+    return PEAK_PARTS_MFMA_TFLOPS if rows == 128 else PEAK_FP32_MFMA_TFLOPS
 
 
 def roofline(flops: int, nbytes: int, seconds: float, workload: str) -> dict:
@@ -952,6 +957,8 @@ def compact(result: dict) -> dict:
     out["mfma_frac"] = _r(result["mfma_frac"])
     rf = result["roofline"]
     out["roofline"] = {k: _r(rf[k]) for k in ("bound", "achieved", "peak", "unit", "frac", "traffic")}
+    if rf["traffic_source"]:  # whether the committed traffic record is of this attention source
+        out["roofline"]["traffic_matches_build"] = rf["traffic_source"]["matches_this_build"]
     if "cpu_baseline" in result:
         cb = result["cpu_baseline"]
         out["cpu_baseline"] = {k: _r(cb[k]) for k in ("value", "unit", "cores", "kind", "sample", "t1_value",

@@ -346,3 +346,15 @@ hipError_t launch_attention(const AttnLaunch &a, hipStream_t stream) {
 }
 
 }  // namespace raya
+
+// The query rows of an item that a launch of these sizes takes (16, 64, or 128 on three-part products),
+// for the tests and the bench's choice of matrix peak; -1 for a head_dim without a kernel.  Row strides
+// short enough for every kernel.
+extern "C" int raya_attention_item_rows(int batch, int heads, int seq, int head_dim, int mask_kind, int mask_arg) {
+    using namespace raya;
+    if (head_dim <= 0 || head_dim > kMaxHeadDim) return -1;
+    AttnLaunch a{};
+    a.batch = batch, a.heads = heads, a.seq = seq, a.head_dim = head_dim;
+    a.mask_kind = mask_kind, a.mask_arg = mask_arg;
+    return (int)item_rows(a, head_dim == 64 || head_dim == 128);
+}

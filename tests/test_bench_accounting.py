@@ -48,3 +48,14 @@ def test_headline_workload_figures():
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, "bench.py", "--gpus", "2"], cwd=ROOT, capture_output=True, text=True)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+def test_matrix_peak_follows_the_librarys_choice(monkeypatch):
+    """Large Block3 grids run on three-part products, the single-tile and small ones on fp32 ones."""
+    monkeypatch.delenv("RAYA_ATTN_ITEMS", raising=False)
+    parts = {n for n in W.ATTENTION if bench.mfma_peak(n) == bench.PEAK_PARTS_MFMA_TFLOPS}
+    assert {"attn_b32_h12_l2048_d64_block3", "attn_b4_h12_l16384_d64_block3"} <= parts
+    assert not parts & {"attn_b32_h12_l2048_d64_blockdiag64", "attn_b4_h12_l16384_d64_blockdiag128",
+                        "attn_b1_h12_l512_d64_block3", "refbench_h16_l8192_d64_window64"}
+    monkeypatch.setenv("RAYA_ATTN_ITEMS", "64")
+    assert bench.mfma_peak("attn_b32_h12_l2048_d64_block3") == bench.PEAK_FP32_MFMA_TFLOPS
