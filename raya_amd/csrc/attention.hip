@@ -103,27 +103,28 @@ constexpr int64_t kSplitBelow = 192;
 // (attention_parts.hip), by the masks and grids where it is the faster one.  Its items are twice
 // as long as the 64-row kernel's, so what it loses is a last round that few of them fill: the
 // grid is measured in rounds of one item a compute unit.  us, 128-row / 64-row / 16-row items:
-// - Full and Block3 at head_dim 64, from 144 items: 16 x 8192 Block3 78 / 112, 4 x 12 x 2048 Full
-//   208 / 322; just past a round (2 x 13 x 1161 Block3, 260 items) 31.6 / 35.1, before it
-//   (2 x 14 x 1109, 252) 22.7 / 35.3.  Fewer items are worth it on one long sequence only (12 x 768,
-//   72 items: 36.7 / 41.6 / 38.2 and 20.6 / 22.1 / 22.1; 12 x 640 31.0 / 34.0 / 24.8); in padded batches
-//   the 16-row items have less to do (3 x 8 x 388 Full 25.7 / 25.2 / 18.3).
+// - Full and Block3 at head_dim 64, from 144 items: 16 x 8192 Block3 80 / 122, 4 x 12 x 2048 Full
+//   193 / 326; just past a round (2 x 13 x 1161 Block3, 260 items) 35.4 / 36.5, before it
+//   (2 x 14 x 1109, 252) 26.0 / 37.2.  Fewer items are worth it on one long sequence only, from 80 (12 x 896,
+//   84 items: Full 42.1 / 49.2 / 43.2, Block3 22.2 / 22.6 / 22.9; 8 x 1152, 72 items: Block3 21.6 / 22.2 / 20.3, Full
+//   51.5 / 57.4 / 52.3; 4 x 2304, 72 items: Full 97.0 / 117 / 95.3; 12 x 640 Full 32.2 / 34.8 / 26.0); in padded
+//   batches the 16-row items have less to do (3 x 8 x 388 Full 27.4 / 27.3 / 24.6).
 // - head_dim 128 (one wave a SIMD: Q's parts and the output alone fill 160 registers): Block3
-//   2 x 8 x 3000 73 / 102, Full 2 x 8 x 2048 185 / 290, from 144 items (Block3 8 x 1536, 96 items,
-//   36.3 / 35.5).  Past one round only where the rounds are 70% full: Full 23 x 3 x 442 (276 items)
-//   87 / 72, Block3 12 x 15 x 227 (360) 52 / 67.
+//   2 x 8 x 3000 79 / 92, Full 2 x 8 x 2048 183 / 290, from 144 items (Block3 8 x 1536, 96 items,
+//   39.0 / 37.1).  Past one round only where the rounds are 70% full: Full 23 x 3 x 442 (276 items)
+//   92 / 73, Block3 12 x 15 x 227 (360) 63 / 67.
 // - Sliding(w) from w = 128: part of an item's keys lie outside each wave's windows.  8 x 12 x 2048
-//   at w = 64 73 / 70, 128 92 / 110, 256 148 / 191; 13 x 8 x 652 at 107 48.4 / 45.6.  Past one
-//   round at 75% (8 x 5 x 1217 at 205, 400 items, 51 / 58).  At head_dim 128 from w = 256, past one round
-//   at 90% (18 x 4 x 541 at 237, 360 items, 87 / 76): 16 x 8 x 1024 of 256 to 1024 valid rows 213 / 228 at
-//   256, but 153 / 142 at 128, and 32 x 12 x 1024 at 128 402 / 383.
+//   at w = 64 77 / 76, 128 106 / 136, 256 172 / 239; 13 x 8 x 652 at 107 54 / 56.  Past one
+//   round at 75% (8 x 5 x 1217 at 205, 400 items, 53 / 62).  At head_dim 128 from w = 256, past one round
+//   at 90% (18 x 4 x 541 at 237, 360 items, 126 / 113): 4 x 8 x 2048 at 256 150 / 169 and 16 x 8 x 1024 of 256
+//   to 1024 valid rows 213 / 228, but at 128 100 / 102 and 153 / 142, and 32 x 12 x 1024 at 128 402 / 383.
 // - not BlockDiag: one or two tiles an item leave nothing to gain from cheaper products (64 is
 //   bound by memory).
 // Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.  The lengths of a
 // device batch are not known here: with valid rows from a quarter to half of seq the 128-row kernel is
 // the faster one too (64 x 12 x 512 of 128 to 256 rows: Full 76 / 109, Block3 78 / 107, Sliding(128)
 // 76 / 99), below an eighth of seq it is not (64 x 12 x 512 of 16 to 32 rows: Full 49 / 37, Sliding(128) 43 / 28).
-constexpr int64_t kPartsFrom = 144, kPartsFromAlone = 72, kAloneSeq = 768;
+constexpr int64_t kPartsFrom = 144, kPartsFromAlone = 80, kAloneSeq = 768;
 constexpr int64_t kPartsWindow = 128, kPartsWindowWide = 256, kRound = 256;
 
 bool takes_parts(const AttnLaunch &a) {

@@ -4,16 +4,16 @@
 // 113 of its 155 TFLOP/s).  Here every operand of both products is the exact sum of three
 // bfloat16 parts and a product the six part products that carry it, as in gemm_kernel.hpp:
 // 6 / 16 of the fp32 instruction's time, fewer roundings, and the probabilities keep all their
-// 24 bits.  Splitting costs 5.5 VALU operations an element, so a workgroup takes 128 rows:
-// each K and V element is split once for all of them, and each wave's 32 rows fill the
-// 32 x 32 x 16 instruction.  At head_dim 64 a wave's tile of 64 keys is 96 matrix instructions (3,072 clocks)
-// and about 500 VALU operations (2,400 at the 4.7 clocks they sustain); two waves a SIMD overlap
-// them to about 3,900 clocks a tile.
+// 24 bits (down to 2^-110 of a row's largest; below, see the checks).  Splitting costs 5.5 VALU
+// operations an element, so a workgroup takes 128 rows: each K and V element is split once for all of
+// them, and each wave's 32 rows fill the 32 x 32 x 16 instruction.  At head_dim 64 a wave's tile of
+// 64 keys is 96 matrix instructions (3,072 clocks) and about 500 VALU operations (2,400 at the 4.7
+// clocks they sustain); two waves a SIMD overlap them to about 3,900 clocks a tile.
 //
-// Measured (us, before on the 64-row fp32 kernel): Block3 16 x 8192 116 -> 77 (165 TFLOP/s),
-// Block3 32 x 12 x 2048 402 -> 300, Full 4 x 12 x 2048 (1024 to 2048 valid) 342 -> 219, Full
-// 1 x 12 x 4096 442 -> 294 (175 TFLOP/s); head_dim 128: Block3 8 x 8 x 2048 228 -> 167, Full
-// 2 x 8 x 2048 290 -> 185 (186 TFLOP/s); relative 2-norm error against float64 4.6e-7 -> 3.9e-7
+// Measured (us, the 64-row fp32 kernel -> this one, on one card): Block3 16 x 8192 119 -> 80 (159 TFLOP/s),
+// Block3 32 x 12 x 2048 610 -> 450, Full 4 x 12 x 2048 (1024 to 2048 valid) 329 -> 194, Full
+// 1 x 12 x 4096 439 -> 303 (170 TFLOP/s); head_dim 128: Block3 8 x 8 x 2048 229 -> 163, Full
+// 2 x 8 x 2048 289 -> 185 (186 TFLOP/s); relative 2-norm error against float64 4.6e-7 -> 3.9e-7
 // (Block3), 7.7e-7 -> 7.0e-7 (Full).
 //
 //   S^T = K Q^T (32 keys x 32 queries per subtile), online softmax as in attention_body.hpp,

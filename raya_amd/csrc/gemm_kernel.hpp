@@ -25,9 +25,9 @@
 // TFLOP/s), so six of them take 6 / 16 of the time.  What bounds the large tiles is the
 // chip's power: the shader clock falls from 2.4 to about 1.75 GHz while they run, and a
 // plain library bfloat16 product reaches 1,430 TFLOP/s (238 in these terms; its fp32 one
-// 155).  At M = 21,405, [N, K] = 2304 x 768: 550 us (138 TFLOP/s) on the fp32 instruction,
-// 367 us (207) here; 768 x 768 189 -> 127 us, GeGLU 6144 x 768 1,463 -> 920 us,
-// 768 x 3072 725 -> 443 us.
+// 155).  At M = 21,405, [N, K] = 2304 x 768: 550-587 us by card (138-129 TFLOP/s) on the fp32
+// instruction, 368-398 (206-190) here; on the slower card 768 x 768 189 -> 129 us, GeGLU
+// 6144 x 768 1,479 -> 929, 768 x 3072 724 -> 448.
 //
 // Parts of Inf and NaN (and of |x| from 2^105 on, whose scaled value is above the largest
 // bfloat16) are not sums of anything, so such an operand leaves every output of its row or column

@@ -271,7 +271,8 @@ def test_longest_first_at_its_limit_and_packed(hip_attention, b, d):
 
 # Batch, heads, seq, head_dim, mask and the item height that a launch takes, on either side of each line.
 CHOICES = [(2, 9, 1024, 64, R.Mask.BLOCK3, "128"), (1, 143, 100, 64, R.Mask.BLOCK3, "64"), (2, 72, 100, 64, R.Mask.FULL, "128"),
-           (1, 12, 768, 64, R.Mask.FULL, "128"), (1, 12, 760, 64, R.Mask.FULL, "16"), (2, 6, 768, 64, R.Mask.FULL, "16"),
+           (1, 12, 896, 64, R.Mask.FULL, "128"), (1, 12, 768, 64, R.Mask.FULL, "16"), (1, 16, 768, 64, R.Mask.BLOCK3, "128"),
+           (1, 16, 760, 64, R.Mask.BLOCK3, "64"), (2, 6, 768, 64, R.Mask.FULL, "16"),
            (1, 12, 768, 128, R.Mask.BLOCK3, "16"), (1, 18, 1024, 128, R.Mask.BLOCK3, "128"),
            (23, 3, 442, 128, R.Mask.FULL, "64"), (23, 4, 442, 128, R.Mask.FULL, "128"),
            (64, 3, 130, 64, R.Mask.BLOCK3, "64"), (64, 3, 200, 64, R.Mask.BLOCK3, "128"),
