@@ -413,9 +413,13 @@ __device__ __forceinline__ void parts_body(const AttnLaunch &a, const Plan &p, c
                 y = make_float4(oacc[t][4 * r] * inv, oacc[t][4 * r + 1] * inv, oacc[t][4 * r + 2] * inv,
                                 oacc[t][4 * r + 3] * inv);
             out_lo = min(min(out_lo, min(small_key(y.x), small_key(y.y))), min(small_key(y.z), small_key(y.w)));
-            out_nan = __builtin_fmaf(y.x, 0.f, __builtin_fmaf(y.y, 0.f, __builtin_fmaf(y.z, 0.f, __builtin_fmaf(y.w, 0.f, out_nan))));
+            out_nan = __builtin_fmaf(y.x, 0.f, __builtin_fmaf(y.y, 0.f, out_nan));
+            out_nan = __builtin_fmaf(y.z, 0.f, __builtin_fmaf(y.w, 0.f, out_nan));
             *(float4 *)(st + li * D + 4 * ((8 * t + 2 * r + h) ^ (li & 15))) = y;
         }
+    // The row's smallest output that is not zero: its dims are in lanes li and li + 32.
+    const auto halves = __builtin_amdgcn_permlane32_swap(out_lo, out_lo, false, false);
+    out_lo = min(halves[0], halves[1]);
     if (!zero_row) bad |= out_lo < small_key(kTinyOut) || out_lo == ~0u || out_nan != 0.f;
     int redo = 0;  // halves
     if (__syncthreads_or(bad || bad_v)) {

@@ -307,3 +307,19 @@ def test_default_dispatch(hip_attention, monkeypatch, b, h, s, d, mask, rows):
         want = oracle.naive_attend(q, k, v, kind, lens[i], R.kernels.default_scale(d), block=block, window=window)
         close(got[i, :, :lens[i]].cpu().numpy(), want[:, :lens[i]])
         assert (got[i, :, lens[i]:] == 0).all()
+
+
+@pytest.mark.parametrize("name", ["block3", "full", "sliding200"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_masks_are_exact(hip_attention, name, d):
+    """V one-hot on key j: exactly the rows that see it get its weight, and the other dims stay zero."""
+    seq, mask = 400, MASKS[name][0]
+    q, k, _ = (torch.from_numpy(t[None]).cuda() for t in inputs(41, 1, seq, d))
+    for j in (0, 63, 64, 127, 128, 255, 256, 399):
+        v = torch.zeros_like(q)
+        v[0, 0, j, j % d] = 1.0
+        out = attend(hip_attention, [q, k, v], [seq], mask)[0, 0].cpu()
+        want = torch.tensor([mask.allows(i, j) for i in range(seq)])
+        assert torch.equal(out[:, j % d] > 0, want)
+        out[:, j % d] = 0
+        assert (out == 0).all()
