@@ -323,3 +323,52 @@ def test_masks_are_exact(hip_attention, name, d):
         assert torch.equal(out[:, j % d] > 0, want)
         out[:, j % d] = 0
         assert (out == 0).all()
+
+
+def test_random_sweep_against_the_oracle(hip_attention):
+    """36 random batched launches: batch 1-4, heads 1-3, seq 1-700, both head dims, every mask with a
+    kernel and windows from 1 to past seq, valid lengths anywhere (clamped into [0, seq] by the entry
+    point), negative and doubled scales."""
+    rng = np.random.default_rng(2025)
+    for case in range(36):
+        b, h, s, d = int(rng.integers(1, 5)), int(rng.integers(1, 4)), int(rng.integers(1, 701)), (64, 128)[case % 2]
+        arg = int(rng.integers(1, s + 80))
+        mask, kind, block, window = [MASKS["block3"], MASKS["full"], (R.Mask.sliding(arg), oracle.MASK_SLIDING, 0, arg)][case % 3]
+        valid = rng.integers(-3, s + 4, size=b).astype(np.int32)
+        clamped = np.clip(valid, 0, s).astype(np.int32)
+        scale = R.kernels.default_scale(d) * float(rng.choice([1.0, -1.0, 2.0]))
+        q, k, v = (rng.standard_normal((b, h, s, d)).astype(np.float32) for _ in range(3))
+        print(f"case {case}: b{b} h{h} s{s} d{d} {mask} valid {valid.tolist()} scale {scale:.4f}", flush=True)
+        want = oracle.naive_attend_batched(q, k, v, kind, clamped, scale, block=block, window=window)
+        out = torch.full((b, h, s, d), float("nan"), device="cuda")
+        hip_attention.attend_batched(*(torch.from_numpy(x).cuda() for x in (q, k, v)), out, torch.from_numpy(valid).cuda(),
+                                     mask, scale=scale)
+        got = out.cpu().numpy()
+        if (clamped > 0).any():
+            close(np.concatenate([got[i, :, :n].reshape(-1) for i, n in enumerate(clamped)]),
+                  np.concatenate([want[i, :, :n].reshape(-1) for i, n in enumerate(clamped)]))
+        for i, n in enumerate(clamped):
+            assert (got[i, :, n:] == 0).all()
+
+
+def test_full_size_block3_by_default_against_float64(hip_attention, monkeypatch):
+    """The 32 x 12 x 2048 Block3 batch (valid lengths 512 to 2048) as a launch takes it by itself, every
+    output against float64 on the device."""
+    monkeypatch.delenv("RAYA_ATTN_ITEMS")
+    b, h, s, d = 32, 12, 2048, 64
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    x = [torch.randn(b, h, s, d, device="cuda", generator=gen) for _ in range(3)]
+    lens = [int(n) for n in synth.integers(77, b, 512, 2048)]
+    out = attend(hip_attention, x, lens, R.Mask.BLOCK3)
+    blk = torch.arange(s, device="cuda") // 128
+    near = (blk[:, None] - blk[None]).abs() <= 1
+    worst = total = norm = 0.0
+    for i, n in enumerate(lens):
+        q, k, v = (t[i, :, :n].double() for t in x)
+        w = torch.softmax((torch.matmul(q, k.transpose(1, 2).contiguous()) * 0.125).masked_fill(~near[:n, :n], -np.inf), -1)
+        want = torch.matmul(w, v)
+        diff = out[i, :, :n].double() - want
+        worst, total, norm = max(worst, float(diff.abs().max())), total + float((diff ** 2).sum()), norm + float((want ** 2).sum())
+        assert (out[i, :, n:] == 0).all()
+    print(f"max-abs {worst:.2e}, rel-L2 {(total / norm) ** 0.5:.2e}")
+    assert worst <= 1e-5 and (total / norm) ** 0.5 <= 1e-6
