@@ -122,8 +122,9 @@ constexpr int64_t kSplitBelow = 192;
 //   bound by memory).
 // Items that hold few rows waste them: 64 x 130 rows Block3 39 / 36, 64 x 100 25 / 34.  The lengths of a
 // device batch are not known here: with valid rows from a quarter to half of seq the 128-row kernel is
-// the faster one too (64 x 12 x 512 of 128 to 256 rows: Full 76 / 109, Block3 78 / 107, Sliding(128)
-// 76 / 99), below an eighth of seq it is not (64 x 12 x 512 of 16 to 32 rows: Full 49 / 37, Sliding(128) 43 / 28).
+// the faster one too (64 x 12 x 512 of 128 to 256 rows: Full 74 / 108, Block3 76 / 108, Sliding(128)
+// 78 / 100), and so with fewer (of 16 to 32: Full 28 / 37, Sliding(128) 25 / 28; 16 x 8 x 1024 of
+// 32 to 64, Full 17.8 / 16.9).
 constexpr int64_t kPartsFrom = 144, kPartsFromAlone = 80, kAloneSeq = 768;
 constexpr int64_t kPartsWindow = 128, kPartsWindowWide = 256, kRound = 256;
 
